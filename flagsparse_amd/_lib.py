@@ -57,6 +57,9 @@ EXPORTED_SYMBOLS = (
     "fs_spmv_noalloc_scratch_bytes",
     "fs_spmv_csr_noalloc",
     "fs_spmv_csr_oneshot",
+    "fs_spmv_scatter_workspace_bytes",
+    "fs_spmv_csr_scatter",
+    "fs_spmv_coo_scatter",
     "fs_spmv_opt_max_buckets",
     "fs_spmv_opt_workspace_bytes",
     "fs_spmv_opt_buckets",
@@ -210,6 +213,14 @@ def _declare(lib):
     lib.fs_spmv_sell.argtypes = [_i32, _i32, _i32, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]
     lib.fs_spmv_csr_oneshot.restype = _i32
     lib.fs_spmv_csr_oneshot.argtypes = [_i32, _i32, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]
+    lib.fs_spmv_scatter_workspace_bytes.restype = _sz
+    lib.fs_spmv_scatter_workspace_bytes.argtypes = [_i32, _i64, _i64]
+    lib.fs_spmv_csr_scatter.restype = _i32
+    lib.fs_spmv_csr_scatter.argtypes = [_i32, _i32, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _sz,
+                                        _vp, _vp]
+    lib.fs_spmv_coo_scatter.restype = _i32
+    lib.fs_spmv_coo_scatter.argtypes = [_i32, _i32, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _sz,
+                                        _vp, _vp]
     lib.fs_spmm_sell.restype = _i32
     lib.fs_spmm_sell.argtypes = [_i32, _i32, _i32, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i64,
                                  _vp]

@@ -23,6 +23,7 @@
 //    through the sort and a gather at the end, the column pointer read off
 //    the sorted keys (radix_* kernels).
 #include "fs_common.hpp"
+#include "radix_tile.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -40,43 +41,6 @@ constexpr int64_t kSub = 64 * kChunks;      // entries per wave sub-tile
 constexpr int kWavesPerBlock = 4;
 constexpr int kScanItems = 16;              // per-thread items in the scan kernels
 constexpr int64_t kScanTile = 256 * kScanItems;
-
-__device__ inline int lane_id_t() {
-  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-}
-__device__ inline int count_below_t(uint64_t mask) {
-  return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
-}
-__device__ inline void wave_sync_t() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Tile of workgroup b out of n so that each of the 8 XCDs (to which
-// workgroups are dealt in turn) walks one contiguous range of tiles: the
-// runs that neighbouring tiles of a scatter write for one digit or panel
-// are adjacent in the output, so they meet in the same L2 and leave it as
-// whole lines.
-__device__ inline int64_t xcd_tile(uint32_t b, uint32_t n) {
-  constexpr uint32_t kXcds = 8;
-  const uint32_t q = n / kXcds, r = n % kXcds, x = b % kXcds, i = b / kXcds;
-  return x < r ? (int64_t)x * (q + 1) + i : (int64_t)r * (q + 1) + (int64_t)(x - r) * q + i;
-}
-
-// Lanes (among `active`) whose digit equals this lane's digit; `mask` has
-// the pass's digit bits (a uniform value: bits above it are skipped).
-__device__ inline uint64_t peer_mask(unsigned digit, uint64_t active, unsigned mask) {
-  uint64_t peers = active;
-#pragma unroll
-  for (int b = 0; b < kRadixBits; ++b) {
-    if (!((mask >> b) & 1u)) break;
-    const bool bit = (digit >> b) & 1u;
-    const uint64_t m = __ballot(bit);
-    peers &= bit ? m : ~m;
-  }
-  return peers;
-}
 
 // Key source: pass 0 reads the CSR column indices directly.
 template <class K>
@@ -97,28 +61,6 @@ __device__ inline void load_tile_keys(const void* keys, int kind, int64_t base, 
     const int64_t e = base + (int64_t)ch * 64 + lane;
     key[ch] = e < n ? load_key<K>(keys, kind, e) : (K)0;
   }
-}
-
-__device__ inline int64_t block_exclusive_scan(int64_t v, int64_t* s_wave, int64_t& total) {
-  const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
-  int64_t x = v;
-  for (int off = 1; off < 64; off <<= 1) {
-    int lo = __builtin_amdgcn_ds_bpermute((lane - off) << 2, (int)(x & 0xffffffff));
-    int hi = __builtin_amdgcn_ds_bpermute((lane - off) << 2, (int)(x >> 32));
-    int64_t y = ((int64_t)hi << 32) | (uint32_t)lo;
-    if (lane >= off) x += y;
-  }
-  if (lane == 63) s_wave[w] = x;
-  __syncthreads();
-  int64_t wave_base = 0;
-  total = 0;
-  for (int k = 0; k < (int)(blockDim.x >> 6); ++k) {
-    if (k < w) wave_base += s_wave[k];
-    total += s_wave[k];
-  }
-  __syncthreads();
-  return wave_base + x - v;
 }
 
 template <class K, class CT>
@@ -263,24 +205,6 @@ constexpr int kScatterFirst = 1;  // payload built from values and row ids
 constexpr int kScatterLast = 2;   // payload out as transposed values / rows
 constexpr int kScatterOnly = 3;   // first and last (a single pass)
 
-// Inclusive max-scan over the wave (DPP row shifts within 16-lane rows,
-// then row broadcasts across them; lanes without a source read 0, the
-// identity of an unsigned max).
-template <int CTRL, int ROWMASK>
-__device__ inline unsigned dpp_shift_u(unsigned v) {
-  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWMASK, 0xF, false);
-}
-__device__ inline unsigned umax_(unsigned a, unsigned b) { return a > b ? a : b; }
-__device__ inline unsigned wave_max_scan(unsigned v) {
-  v = umax_(v, dpp_shift_u<0x111, 0xF>(v));  // row_shr:1
-  v = umax_(v, dpp_shift_u<0x112, 0xF>(v));  // row_shr:2
-  v = umax_(v, dpp_shift_u<0x114, 0xF>(v));  // row_shr:4
-  v = umax_(v, dpp_shift_u<0x118, 0xF>(v));  // row_shr:8
-  v = umax_(v, dpp_shift_u<0x142, 0xA>(v));  // row_bcast:15 -> rows 1, 3
-  v = umax_(v, dpp_shift_u<0x143, 0xC>(v));  // row_bcast:31 -> rows 2, 3
-  return v;
-}
-
 // Row marks of a sub-tile (kSub entries from `base`, rows r0..r1 touching
 // it): every row that starts inside the tile marks its first entry with
 // r - r0 in s_mark (rows read with unit stride, empty rows mark nothing).
@@ -381,7 +305,7 @@ __global__ __launch_bounds__(64, 2) void radix_scatter_kernel(const void* __rest
     const bool valid = ch * 64 + lane < cnt;
     const uint64_t active = __ballot(valid);
     const unsigned digit = (unsigned)(key[ch] >> shift) & mask;
-    const uint64_t peers = peer_mask(digit, active, mask);
+    const uint64_t peers = match_lanes<kRadixBits>(digit, active, mask);
     const int rank = count_below_t(peers);
     unsigned old = 0;
     if (valid && rank == 0) old = atomicAdd(&s_cnt[digit], (unsigned)__popcll(peers));
@@ -733,48 +657,6 @@ __global__ __launch_bounds__(256) void identity_kernel(const void* __restrict__ 
   if (k < n) keys[k] = load_key<K>(cols, kind, k);
 }
 
-// ---- workgroup-tile radix passes (the transpose of 4- and 8-byte values) ----
-// A workgroup of kWgWaves waves sorts a tile of kWgTile entries per pass
-// (wave w holds entries [w * kWgSub, (w + 1) * kWgSub) of the tile in
-// registers, kWgChunks per lane, and ranks them as radix_scatter_kernel
-// does, against its own LDS counters).  The larger tile allows more digits
-// at the same run length per digit, up to 11 key bits per pass: the 20-bit
-// columns of a 1M-column matrix take two passes instead of three.  The
-// payload carries the entry's value and row (an 8-byte word for 4-byte
-// values, 12 bytes for 8-byte values), built by the first pass from the
-// CSR arrays and written out as the transposed values and rows by the last,
-// and the last pass writes no keys: the column pointer comes from an atomic
-// minimum of the first position of each column the tile holds, and a
-// suffix minimum over the columns (empty columns take the next one's start).
-#ifndef FS_WG_WAVES
-#define FS_WG_WAVES 8
-#endif
-#ifndef FS_WG_CHUNKS
-#define FS_WG_CHUNKS 12
-#endif
-#ifndef FS_WG_MIN_WAVES
-#define FS_WG_MIN_WAVES 4
-#endif
-constexpr int kWgWaves = FS_WG_WAVES;
-constexpr int kWgThreads = 64 * kWgWaves;
-constexpr int kWgChunks = FS_WG_CHUNKS;
-constexpr int64_t kWgSub = 64 * kWgChunks;
-constexpr int64_t kWgTile = kWgWaves * kWgSub;
-constexpr int kWgMaxBits = 11;
-constexpr int kWgScanTiles = 16;  // tiles per block of the digit scan
-constexpr int kWgMaxDigits = 1 << kWgMaxBits;
-// staging buffer: row marks, wave counters, keys, then the payload in
-// windows (a multiple of 8 and 12 bytes; half a tile of 12-byte payload, so
-// the payload leaves in two windows)
-constexpr int kWgBufHalf = (int)(kWgTile / 2) * 12;
-constexpr int kWgBufMin = kWgWaves * kWgMaxDigits * 2 > kWgBufHalf ? kWgWaves * kWgMaxDigits * 2 : kWgBufHalf;
-constexpr int kWgBufBytes = (kWgBufMin + 23) / 24 * 24;
-// the wave counters hold two digits per word (16-bit counts: a wave ranks
-// at most kWgSub entries, a tile at most kWgTile < 2^16)
-static_assert(kWgTile < 65536, "16-bit digit counters");
-static_assert(kWgWaves * kWgMaxDigits * 2 <= kWgBufBytes, "wave counters fit the staging buffer");
-static_assert(kWgTile * 4 <= kWgBufBytes, "row marks and keys fit the staging buffer");
-
 // The payload between passes: the entry's value word(s) and row.  (Records
 // that also carried the key, so that a digit's run left as one block, measured
 // slower: the next pass's count then reads the whole records.)
@@ -810,51 +692,6 @@ struct WgIO {
   int other64;
   int swap;                 // this pass sorts by the payload's index: it and the key change places
 };
-
-// Keys of a wave sub-tile: `cnt` entries from `base` (kind 1: 8-byte
-// column indices below 2^32; otherwise 4-byte keys); one per-lane base
-// pointer, the chunks at immediate offsets from it.
-__device__ inline void wg_load_keys(const void* keys, int kind, int64_t base, int cnt, int lane,
-                                    uint32_t (&key)[kWgChunks]) {
-  if (kind == 5 || kind == 6) {  // one word of each 8- / 12-byte payload (`keys` points at it)
-    const int W = kind == 5 ? 2 : 3;
-    const uint32_t* p = static_cast<const uint32_t*>(keys) + (base + lane) * W;
-#pragma unroll
-    for (int ch = 0; ch < kWgChunks; ++ch) key[ch] = ch * 64 + lane < cnt ? p[ch * 64 * W] : 0u;
-  } else if (kind == 1) {
-    const int64_t* p = static_cast<const int64_t*>(keys) + base + lane;
-#pragma unroll
-    for (int ch = 0; ch < kWgChunks; ++ch) key[ch] = ch * 64 + lane < cnt ? (uint32_t)p[ch * 64] : 0u;
-  } else {
-    const uint32_t* p = static_cast<const uint32_t*>(keys) + base + lane;
-#pragma unroll
-    for (int ch = 0; ch < kWgChunks; ++ch) key[ch] = ch * 64 + lane < cnt ? p[ch * 64] : 0u;
-  }
-}
-
-// Row of every entry of a wave sub-tile (rows r0..r1 touch it): each row
-// starting inside marks its first entry with r - r0, and a wave max-scan
-// carried across the chunks gives entry j the largest mark at or before j.
-template <class P>
-__device__ inline void wg_rows(const P* __restrict__ rowptr, int64_t r0, int64_t r1, int64_t base, int cnt,
-                               unsigned* s_mark, int lane, uint32_t (&row)[kWgChunks]) {
-  for (int j = lane; j < (int)kWgSub; j += 64) s_mark[j] = 0u;
-  wave_sync_t();
-  for (int64_t r = r0 + 1 + lane; r <= r1; r += 64) {
-    const int64_t st = (int64_t)rowptr[r];
-    // (st >= base on a valid row pointer; the test keeps a malformed one,
-    // which the caller's structure check reports, inside the tile's marks)
-    if (st >= base && st - base < cnt && (int64_t)rowptr[r + 1] > st) s_mark[st - base] = (unsigned)(r - r0);
-  }
-  wave_sync_t();
-  unsigned carry = 0u;
-#pragma unroll
-  for (int ch = 0; ch < kWgChunks; ++ch) {
-    const unsigned m = umax_(wave_max_scan(s_mark[ch * 64 + lane]), carry);
-    carry = (unsigned)__builtin_amdgcn_readlane((int)m, 63);
-    row[ch] = (uint32_t)(r0 + (int64_t)m);
-  }
-}
 
 // Row of the first entry of every wave sub-tile: thread r writes r for the
 // sub-tiles whose first entry lies in row r (one coalesced pass over the row
@@ -988,78 +825,6 @@ __global__ __launch_bounds__(kWgThreads) void wg_count_kernel(const void* __rest
   for (int d = threadIdx.x; d < nd; d += kWgThreads) counts[tile * nd + d] = s_hist[d];
 }
 
-// Exclusive scan of cnt[tile][d] in (digit, tile) order (nd digits, up to
-// kWgMaxDigits): per-block digit sums over kWgScanTiles tiles, one
-// workgroup per digit scanning its block sums, then the downsweep.
-__global__ __launch_bounds__(256) void wg_scan_reduce_kernel(const uint32_t* __restrict__ cnt, int64_t n_tiles,
-                                                             int nd, uint32_t* __restrict__ partial) {
-  const int64_t s0 = (int64_t)blockIdx.x * kWgScanTiles;
-  const int64_t s1 = s0 + kWgScanTiles < n_tiles ? s0 + kWgScanTiles : n_tiles;
-  for (int d = threadIdx.x; d < nd; d += 256) {
-    uint32_t sum = 0;
-    for (int64_t s = s0; s < s1; s += kScanBatch) {
-      uint32_t v[kScanBatch];
-#pragma unroll
-      for (int k = 0; k < kScanBatch; ++k) v[k] = s + k < s1 ? cnt[(s + k) * nd + d] : 0u;
-#pragma unroll
-      for (int k = 0; k < kScanBatch; ++k) sum += v[k];
-    }
-    partial[(int64_t)blockIdx.x * nd + d] = sum;
-  }
-}
-
-__global__ __launch_bounds__(256) void wg_scan_column_kernel(uint32_t* __restrict__ partial, int64_t n_blocks, int nd,
-                                                             uint32_t* __restrict__ totals) {
-  __shared__ int64_t s_wave[4];
-  const int d = blockIdx.x;
-  int64_t carry = 0;
-  for (int64_t b0 = 0; b0 < n_blocks; b0 += 256) {
-    const int64_t b = b0 + threadIdx.x;
-    const int64_t v = b < n_blocks ? (int64_t)partial[b * nd + d] : 0;
-    int64_t sum;
-    const int64_t ex = block_exclusive_scan(v, s_wave, sum);
-    if (b < n_blocks) partial[b * nd + d] = (uint32_t)(carry + ex);
-    carry += sum;
-  }
-  if (threadIdx.x == 0) totals[d] = (uint32_t)carry;
-}
-
-__global__ __launch_bounds__(256) void wg_scan_down_kernel(uint32_t* __restrict__ cnt, int64_t n_tiles, int nd,
-                                                           const uint32_t* __restrict__ partial,
-                                                           const uint32_t* __restrict__ totals) {
-  __shared__ int64_t s_wave[4];
-  __shared__ uint32_t s_base[kWgMaxDigits];
-  // digit starts: thread t scans digits [t q, t q + q)
-  const int q = (nd + 255) / 256;
-  const int d0 = threadIdx.x * q;
-  int64_t mine = 0;
-  for (int j = 0; j < q; ++j)
-    if (d0 + j < nd) mine += totals[d0 + j];
-  int64_t all;
-  int64_t run = block_exclusive_scan(mine, s_wave, all);
-  for (int j = 0; j < q; ++j)
-    if (d0 + j < nd) {
-      s_base[d0 + j] = (uint32_t)run;
-      run += totals[d0 + j];
-    }
-  __syncthreads();
-  const int64_t s0 = (int64_t)blockIdx.x * kWgScanTiles;
-  const int64_t s1 = s0 + kWgScanTiles < n_tiles ? s0 + kWgScanTiles : n_tiles;
-  for (int d = threadIdx.x; d < nd; d += 256) {
-    uint32_t r = s_base[d] + partial[(int64_t)blockIdx.x * nd + d];
-    for (int64_t s = s0; s < s1; s += kScanBatch) {
-      uint32_t v[kScanBatch];
-#pragma unroll
-      for (int k = 0; k < kScanBatch; ++k) v[k] = s + k < s1 ? cnt[(s + k) * nd + d] : 0u;
-#pragma unroll
-      for (int k = 0; k < kScanBatch; ++k) {
-        if (s + k < s1) cnt[(s + k) * nd + d] = r;
-        r += v[k];
-      }
-    }
-  }
-}
-
 // Stable scatter of one workgroup-tile pass (see above).  Steps: keys and
 // payload into registers; per wave, ranks within the digit against the
 // wave's LDS counters (16-bit, two digits per word); per digit, the waves'
@@ -1159,14 +924,7 @@ __global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel
     const bool valid = ch * 64 + lane < cnt;
     const uint64_t active = __ballot(valid);
     const unsigned digit = (key[ch] >> shift) & mask;
-    uint64_t peers = active;
-#pragma unroll
-    for (int b = 0; b < kWgMaxBits; ++b) {
-      if (!((mask >> b) & 1u)) break;
-      const bool bit = (digit >> b) & 1u;
-      const uint64_t m = __ballot(bit);
-      peers &= bit ? m : ~m;
-    }
+    const uint64_t peers = match_lanes<kWgMaxBits>(digit, active, mask);
     const int rank = count_below_t(peers);
     const unsigned half = (digit & 1u) * 16u;
     unsigned old = 0;
@@ -1257,8 +1015,7 @@ __global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel
   __syncthreads();
   // the payload, in windows of the buffer (each window holds whole rounds
   // of sorted positions, so a thread's positions stay its own)
-  constexpr int kWin = kWgBufBytes / (int)sizeof(Pay);
-  static_assert(kWin % kWgThreads == 0, "windows hold whole rounds of sorted positions");
+  constexpr int kWin = kWgBufBytes / (int)sizeof(Pay) / kWgThreads * kWgThreads;
   Pay* s_pay = reinterpret_cast<Pay*>(s_buf);
   for (int w0 = 0; w0 < tcnt; w0 += kWin) {
 #pragma unroll

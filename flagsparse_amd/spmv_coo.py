@@ -9,7 +9,8 @@ pointer of the sorted entries, so a launch is one call of the CSR SpMV
 kernels: nnz-balanced, short rows and power-law rows alike, no atomics and
 bit-reproducible run to run.  ``sort_by_row=False`` keeps the caller's
 order in the prepared fields (as the reference does) and still computes
-through the sorted copy.
+through the sorted copy.  An unprepared call sorts nothing: its products are
+scattered by output (``fs_spmv_coo_scatter``).
 
 Public surface, argument meaning and error messages follow the reference:
   prepare_spmv_coo / PreparedCoo         spmv_coo.py:77-135, 425-474
@@ -25,9 +26,10 @@ import time
 
 import torch
 
-from ._common import _INDEX_LIMIT_INT32, SUPPORTED_INDEX_DTYPES
+from . import _lib
+from ._common import _INDEX_LIMIT_INT32, HIP_VALUE_DTYPES, SUPPORTED_INDEX_DTYPES
 from .coo import coo_to_csr_for_spmv
-from .spmv_csr import _hip_spmv_csr_impl_prepared, _prepare_spmv
+from .spmv_csr import _hip_spmv_csr_impl_prepared, _oneshot_flags, _prepare_spmv
 
 SUPPORTED_SPMV_COO_VALUE_DTYPES = (
     torch.float32,
@@ -250,12 +252,16 @@ class _PreparedCooLaunch:
         "index_fallback_reason",
         "sorted",
         "conj",
+        "bad_indices",
     )
 
+    # sorted_coo: the sorted orientation, or None for a launch over the caller's
+    # unsorted entries, which leaves (bad row, bad col) in bad_indices.
     def __init__(self, sorted_coo, data, row, col, shape, seg_starts=None, op=SPMV_COO_OP_NON, conj=False,
                  index_fallback_policy="auto", index_fallback_applied=False, index_fallback_reason=None):
         self.sorted = sorted_coo
         self.conj = bool(conj)
+        self.bad_indices = None
         self.data = data
         self.row = row
         self.col = col
@@ -326,7 +332,10 @@ def _validate_x_coo(x, launch):
 
 def _hip_spmv_coo_kernel(launch, x, block_size, num_warps, block_inner):
     """One launch (replaces _triton_spmv_coo_kernel, spmv_coo.py:575-644): the
-    CSR SpMV kernels over the sorted entries of the launch's orientation."""
+    CSR SpMV kernels over the sorted entries of the launch's orientation, or
+    the scattered products of unsorted ones."""
+    if launch.sorted is None:
+        return _hip_spmv_coo_scatter(launch, x)
     if launch.n_rows == 0:
         return torch.zeros(0, dtype=launch.data.dtype, device=launch.data.device)
     return _hip_spmv_csr_impl_prepared(launch.sorted.csr(conj=launch.conj), x)
@@ -364,7 +373,7 @@ def _spmv_coo_prepared_with_int32_indices(launch, reason):
         raise RuntimeError(f"native int64 COO SpMV failed and int32 fallback is unsafe: {blocker}")
     seg = None if launch.seg_starts is None else launch.seg_starts.to(torch.int32).contiguous()
     srt = launch.sorted
-    sorted32 = _SortedCoo(srt.data, srt.row.to(torch.int32), srt.col.to(torch.int32),
+    sorted32 = None if srt is None else _SortedCoo(srt.data, srt.row.to(torch.int32), srt.col.to(torch.int32),
                           None if srt.seg_starts is None else srt.seg_starts.to(torch.int32), srt.indptr.to(torch.int32),
                           srt.shape)
     return _PreparedCooLaunch(sorted32, launch.data, launch.row.to(torch.int32).contiguous(),
@@ -381,7 +390,9 @@ def _run_spmv_coo_prepared_with_fallback(launch, x, block_size, num_warps, block
         if launch.index_fallback_policy != "auto" or not _spmv_coo_uses_int64_indices(launch):
             raise
         fallback = _spmv_coo_prepared_with_int32_indices(launch, exc)
-        return _hip_spmv_coo_kernel(fallback, x, block_size, num_warps, block_inner)
+        y = _hip_spmv_coo_kernel(fallback, x, block_size, num_warps, block_inner)
+        launch.bad_indices = fallback.bad_indices
+        return y
 
 
 def flagsparse_spmv_coo(
@@ -414,6 +425,11 @@ def flagsparse_spmv_coo(
     if prepared is None:
         if any(a is None for a in (data, row, col, x, shape)):
             raise ValueError("data, row, col, x, shape required when prepared is None")
+        done = _spmv_coo_unsorted(data, row, col, x, shape, op_code, block_size, num_warps, block_inner,
+                                  index_fallback_policy, return_time)
+        if done is not None:
+            y = _finish_spmv_coo(done[0], out)
+            return (y, done[1]) if return_time else y
         prepared = prepare_spmv_coo(data, row, col, shape, sort_by_row=sort_by_row, transpose=transpose_flag, op=op,
                                     index_fallback_policy=index_fallback_policy)
         for srt in (prepared._sorted_non, prepared._sorted_trans):
@@ -447,14 +463,84 @@ def flagsparse_spmv_coo(
     if return_time:
         torch.cuda.synchronize()
         elapsed_ms = (time.perf_counter() - t0) * 1000.0
-    if out is not None:
-        if out.shape != y.shape or out.dtype != y.dtype:
-            raise ValueError("out shape/dtype must match result")
-        out.copy_(y)
-        y = out
+    y = _finish_spmv_coo(y, out)
     if return_time:
         return y, elapsed_ms
     return y
+
+
+def _finish_spmv_coo(y, out):
+    if out is None:
+        return y
+    if out.shape != y.shape or out.dtype != y.dtype:
+        raise ValueError("out shape/dtype must match result")
+    out.copy_(y)
+    return out
+
+
+def _hip_spmv_coo_scatter(launch, x):
+    """One fs_spmv_coo_scatter call over a launch's unsorted entries."""
+    lib = _lib.lib()
+    val_t = _lib.value_code(launch.data.dtype)
+    device = launch.data.device
+    y = torch.empty(launch.n_rows, dtype=launch.data.dtype, device=device)
+    ws = _lib.workspace(lib.fs_spmv_scatter_workspace_bytes(val_t, launch.n_rows, launch.nnz), device)
+    flags = _oneshot_flags()
+    _lib.check(
+        lib.fs_spmv_coo_scatter(
+            val_t, _lib.index_code(launch.row.dtype), _lib.index_code(launch.col.dtype), launch.n_rows, launch.n_cols,
+            launch.nnz, _lib.ptr(launch.data), _lib.ptr(launch.row), _lib.ptr(launch.col), 1 if launch.conj else 0,
+            _lib.ptr(x), _lib.ptr(y), _lib.ptr(ws), ws.numel(), flags.data_ptr(), _lib.stream_handle(device),
+        ),
+        "fs_spmv_coo_scatter",
+    )
+    launch.bad_indices = flags.tolist()[:2]
+    return y
+
+
+def _spmv_coo_unsorted(data, row, col, x, shape, op_code, block_size, num_warps, block_inner, index_fallback_policy,
+                       timed):
+    """The unprepared product without a sort: products scattered by output,
+    the index ranges checked by the kernels and the reference's error
+    (spmv_coo.py:390-422) raised before y is returned.  Returns (y, ms or
+    None), or None when the general path must run: anything it would refuse,
+    empty shapes, float16 / bfloat16, or sizes the scatter does not take."""
+    if not all(torch.is_tensor(t) for t in (data, row, col, x)):
+        return None
+    n_rows, n_cols = int(shape[0]), int(shape[1])
+    transposes = _spmv_coo_op_transposes(op_code)
+    n_out, n_x = (n_cols, n_rows) if transposes else (n_rows, n_cols)
+    if (
+        str(index_fallback_policy).lower() not in ("auto", "strict")
+        or data.dtype not in HIP_VALUE_DTYPES
+        or any(t.ndim != 1 or not t.is_cuda or t.device != data.device for t in (data, row, col, x))
+        or any(t.dtype not in SUPPORTED_INDEX_DTYPES for t in (row, col))
+        or not (data.numel() == row.numel() == col.numel())
+        or x.dtype != data.dtype
+        or x.numel() != n_x
+        or not 0 < min(n_rows, n_cols) <= max(n_rows, n_cols) <= _INDEX_LIMIT_INT32
+        or num_warps not in (1, 2, 4, 8, 16, 32)
+        or block_inner <= 0
+        or (block_inner & (block_inner - 1)) != 0
+        or _lib.lib().fs_spmv_scatter_workspace_bytes(_lib.value_code(data.dtype), n_out, data.numel()) == 0
+    ):
+        return None
+    out_idx, x_idx = (col, row) if transposes else (row, col)
+    launch = _PreparedCooLaunch(None, data.contiguous(), out_idx.contiguous(), x_idx.contiguous(), (n_out, n_x),
+                                op=op_code, conj=op_code == SPMV_COO_OP_CONJ_TRANS and data.dtype.is_complex,
+                                index_fallback_policy=index_fallback_policy)
+    x = x.contiguous()
+    if timed:
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+    y = _run_spmv_coo_prepared_with_fallback(launch, x, block_size, num_warps, block_inner)
+    elapsed_ms = (time.perf_counter() - t0) * 1000.0 if timed else None  # (the call synchronises)
+    bad_row, bad_col = reversed(launch.bad_indices) if transposes else launch.bad_indices
+    if bad_row:
+        raise IndexError("row indices out of range")
+    if bad_col:
+        raise IndexError("col indices out of range")
+    return y, elapsed_ms
 
 
 __all__ = ["PreparedCoo", "prepare_spmv_coo", "flagsparse_spmv_coo", "SUPPORTED_SPMV_COO_VALUE_DTYPES"]

@@ -1241,13 +1241,15 @@ def _oneshot_launch(data, indices, indptr, x, y, n_rows, n_cols, flags):
 
 
 def _spmv_transposed_oneshot(data, indices, indptr, x, shape, op_code, index_fallback_policy):
-    """The unprepared y = A^T x / A^H x with one synchronisation: the
-    structure check (fs_csr_check_enqueue), the transpose (which stays in
-    bounds on any input, fs_csr_transpose_bounded) and the one-launch SpMV
-    on A^T are queued back to back; the reference's structure error, if any,
-    is raised before y is returned (spmv_csr.py:546-558, then the transpose
-    of :477-515 and :615-618).  None when the general path must run: an
-    invalid x, empty shapes, float16 / bfloat16 / complex128, a forced
+    """The unprepared y = A^T x / A^H x with one synchronisation; the
+    reference's structure error, if any, is raised before y is returned
+    (spmv_csr.py:546-558, then the transpose of :477-515 and :615-618).
+    Products scattered by output (fs_spmv_csr_scatter) where its sizes fit
+    (up to 2^23 columns, 2^22 for complex128); beyond, the transpose, which
+    stays in bounds on any input and runs the structure check in its passes
+    (fs_csr_transpose_checked), and the one-launch SpMV on A^T queued behind
+    it.  None when the general path must run: an invalid x, empty shapes,
+    float16 / bfloat16, complex128 beyond the scatter's sizes, a forced
     kernel or a failed launch."""
     if os.environ.get("FLAGSPARSE_SPMV_ONESHOT", "1") == "0" or os.environ.get("FLAGSPARSE_SPMV_KERNEL"):
         return None
@@ -1259,6 +1261,19 @@ def _spmv_transposed_oneshot(data, indices, indptr, x, shape, op_code, index_fal
         x = _validate_spmv_x_for(x, data.dtype, n_rows, data.device)
     except (TypeError, ValueError):
         return None
+    lib = _lib.lib()
+    ws_bytes = lib.fs_spmv_scatter_workspace_bytes(_lib.value_code(data.dtype), n_cols, nnz)
+    if ws_bytes > 0:
+        y = torch.empty(n_cols, dtype=data.dtype, device=data.device)
+        flag_t = _oneshot_flags()
+        ws = _lib.workspace(ws_bytes, data.device)
+        rc = lib.fs_spmv_csr_scatter(
+            _lib.value_code(data.dtype), _lib.index_code(indices.dtype), _lib.index_code(indptr.dtype), n_rows, n_cols,
+            nnz, _lib.ptr(data), _lib.ptr(indices), _lib.ptr(indptr), 1 if op_code == SPMV_OP_CONJ_TRANS else 0,
+            _lib.ptr(x), _lib.ptr(y), _lib.ptr(ws), ws_bytes, flag_t.data_ptr(), _lib.stream_handle(data.device))
+        if rc == 0:
+            _raise_oneshot_flags(flag_t.tolist())
+            return y
     if not _lib.lib().fs_csr_transpose_bounded(_lib.value_code(data.dtype), n_rows, n_cols, nnz):
         return None
     pending = _PendingCheck(data, indices, indptr, n_cols, _SPMV_STRUCT_MESSAGES, lazy=True)
@@ -1302,7 +1317,12 @@ def _spmv_oneshot(data, indices, indptr, x, shape, index_fallback_policy, timed)
     if rc != 0:
         return None
     compute_ms = (time.perf_counter() - t0) * 1000.0 if timed else None
-    flags = flag_t.tolist()
+    _raise_oneshot_flags(flag_t.tolist())
+    return y, compute_ms
+
+
+def _raise_oneshot_flags(flags):
+    """The reference's structure errors, in its order, from a one-launch call's flags."""
     if flags[0]:
         raise ValueError(_SPMV_STRUCT_MESSAGES["start"])
     if flags[1]:
@@ -1311,4 +1331,3 @@ def _spmv_oneshot(data, indices, indptr, x, shape, index_fallback_policy, timed)
         raise ValueError(_SPMV_STRUCT_MESSAGES["monotone"])
     if flags[3]:
         raise IndexError("indices out of range for n_cols")
-    return y, compute_ms

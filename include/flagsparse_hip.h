@@ -210,6 +210,35 @@ int fs_spmv_csr_oneshot(int val_t, int idx_t, int ptr_t, int64_t n_rows, int64_t
                         const void* x, void* y, int32_t* flags, hipStream_t stream);
 
 /*
+ * y = A^T x (conj: A^H x) of a CSR matrix without its transpose, and y += a x
+ * over COO entries in any order, by scattered products: every product goes
+ * to the bucket of its output (2^k consecutive outputs), then each bucket is
+ * summed in a fixed order (the same bits on every run, no atomics on values).
+ * The first replaces the transpose (spmv_csr.py:477-515) and launch
+ * (:679-723) of an unprepared flagsparse_spmv_csr with op = trans / conj; the
+ * second the sorts (spmv_coo.py:425-474) and launch (:575-644) of an
+ * unprepared flagsparse_spmv_coo: entry e adds vals[e] * x[x_idx[e]]
+ * (conjugated values with conj) to y[out_idx[e]].
+ * x has n_rows (n_x) entries, y n_cols (n_out).  flags as for
+ * fs_spmv_csr_oneshot (pinned, zeroed here, written by the kernels, valid on
+ * return: the calls synchronise `stream`): CSR [0..3] a bad start, a bad end,
+ * a decrease, a column out of range; COO [0] an out_idx and [1] an x_idx out
+ * of range.  Any input is computed in bounds; y is garbage when a flag is set.
+ * ws: fs_spmv_scatter_workspace_bytes(val_t, outputs, nnz) bytes, which is 0
+ * for sizes these calls do not take (more than 2^22 outputs for complex128,
+ * 2^23 otherwise, or nnz near 2^32).
+ */
+size_t fs_spmv_scatter_workspace_bytes(int val_t, int64_t n_out, int64_t nnz);
+int fs_spmv_csr_scatter(int val_t, int idx_t, int ptr_t, int64_t n_rows, int64_t n_cols,
+                        int64_t nnz, const void* vals, const void* cols, const void* indptr,
+                        int conj, const void* x, void* y, void* ws, size_t ws_bytes,
+                        int32_t* flags, hipStream_t stream);
+int fs_spmv_coo_scatter(int val_t, int out_idx_t, int x_idx_t, int64_t n_out, int64_t n_x,
+                        int64_t nnz, const void* vals, const void* out_idx, const void* x_idx,
+                        int conj, const void* x, void* y, void* ws, size_t ws_bytes,
+                        int32_t* flags, hipStream_t stream);
+
+/*
  * fs_spmv_csr without a caller workspace, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  The
