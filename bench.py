@@ -311,7 +311,11 @@ def run_config(name, args):
             if sell.table is not None:
                 extra["sell_distinct_offsets"] = sell.n_codes
         pan = prep._panels
-        if pan is not None:
+        if pan is not None and hasattr(pan, "place"):
+            # two-phase gather: the timed call is the whole sequence (gather, region walk, fixup)
+            kernel_call = lambda: (pan.spmv(x, y), 0)[1]  # noqa: E731
+            extra["n_slices"] = pan.n_panels
+        elif pan is not None:
             # column panels: the timed call is the whole panel sequence
             # (block table, panel merge, fixup, panel reduction)
             args_abi = (
@@ -512,7 +516,8 @@ def _gather_floor_spmv(name, cfg, args, lib, device, stream):
     """SpMV: the x gathers alone, in the order the prepared kernel reads them
     (panel by panel for a column-panelled matrix, one launch per panel, so a
     launch's footprint is one x slice as in the panel kernel), and in plain
-    CSR order in one launch."""
+    CSR order in one launch (the only order for a matrix on the two-phase
+    gather, which reads x from LDS)."""
     import torch
 
     import flagsparse_amd as fs
@@ -532,7 +537,7 @@ def _gather_floor_spmv(name, cfg, args, lib, device, stream):
 
     calls = []
     pan = prep._panels
-    if pan is not None:
+    if pan is not None and not hasattr(pan, "place"):
         pn = [int(pan.panel_nnz[q]) for q in range(pan.n_panels + 1)]
         isz = pan.indices.element_size()
         calls = [launcher(_lib.index_code(pan.indices.dtype), pan.indices.data_ptr(), isz, pn[q], pn[q + 1])

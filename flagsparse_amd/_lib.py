@@ -57,6 +57,12 @@ EXPORTED_SYMBOLS = (
     "fs_spmv_noalloc_scratch_bytes",
     "fs_spmv_csr_noalloc",
     "fs_spmv_csr_oneshot",
+    "fs_spmv_gather_slices",
+    "fs_spmv_gather_plan_bytes",
+    "fs_spmv_gather_count",
+    "fs_spmv_gather_fill",
+    "fs_spmv_gather_workspace_bytes",
+    "fs_spmv_csr_gather",
     "fs_spmv_scatter_workspace_bytes",
     "fs_spmv_csr_scatter",
     "fs_spmv_coo_scatter",
@@ -213,6 +219,19 @@ def _declare(lib):
     lib.fs_spmv_sell.argtypes = [_i32, _i32, _i32, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]
     lib.fs_spmv_csr_oneshot.restype = _i32
     lib.fs_spmv_csr_oneshot.argtypes = [_i32, _i32, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]
+    lib.fs_spmv_gather_slices.restype = _i32
+    lib.fs_spmv_gather_slices.argtypes = [_i32, _i64, _i64, _i64, ctypes.POINTER(_i64)]
+    lib.fs_spmv_gather_plan_bytes.restype = _sz
+    lib.fs_spmv_gather_plan_bytes.argtypes = [_i32, _i64, _i64, _i64]
+    lib.fs_spmv_gather_count.restype = _i32
+    lib.fs_spmv_gather_count.argtypes = [_i32, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]
+    lib.fs_spmv_gather_fill.restype = _i32
+    lib.fs_spmv_gather_fill.argtypes = [_i32, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]
+    lib.fs_spmv_gather_workspace_bytes.restype = _sz
+    lib.fs_spmv_gather_workspace_bytes.argtypes = [_i32, _i64, _i64, _i64]
+    lib.fs_spmv_csr_gather.restype = _i32
+    lib.fs_spmv_csr_gather.argtypes = [_i32, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                       _i64, _i64, _vp, _sz, _vp]
     lib.fs_spmv_scatter_workspace_bytes.restype = _sz
     lib.fs_spmv_scatter_workspace_bytes.argtypes = [_i32, _i64, _i64]
     lib.fs_spmv_csr_scatter.restype = _i32

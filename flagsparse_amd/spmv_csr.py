@@ -198,6 +198,16 @@ class PreparedCsrSpmv:
                     torch.cuda.empty_cache()
             if self._sell is not None:
                 return self._plan  # the copy needs no partition or carry
+            worth = _spmv_gather_worth(p, data.element_size(), self._one_shot)
+            if worth is not None:
+                try:
+                    self._panels = GatheredCsr.build(data, self.kernel_indices, self.kernel_indptr, self.n_rows,
+                                                     self.n_cols, self._plan, worth)
+                except torch.OutOfMemoryError:
+                    self._panels = None
+                    torch.cuda.empty_cache()
+                if self._panels is not None:
+                    return self._plan
             if p.kernel == _lib.FS_KERNEL_MERGE:
                 n_panels = _spmv_panel_count(p, data.dtype, self._one_shot)
                 if n_panels > 1:
@@ -239,7 +249,9 @@ class PreparedCsrSpmv:
         return "panel" if self._panels is not None else plan.kernel_name
 
 
-# Column panels pay off once x is larger than an XCD's 4 MiB L2: the random
+# Column panels (matrices that the two-phase gather below does not take:
+# complex128, columns beyond its slices) pay off once x is larger than an XCD's
+# 4 MiB L2: the random
 # gather rate measured on MI355X drops from ~150-190 to ~70 gathers/ns when
 # x (16.8 MB) no longer fits.  A panel slice of up to ~4.5 MiB measured best
 # (4 panels on a 16.8 MB x: 0.61 ms against 0.67 ms with 8 and 1.01 ms with
@@ -269,6 +281,49 @@ def _spmv_panel_count(plan, dtype, one_shot=False):
     while n_panels < 8 and x_bytes > _PANEL_SLICE_BYTES * n_panels:
         n_panels *= 2
     return n_panels if nnz >= 2 * n_panels * n_rows else 0
+
+
+# The two-phase gather (GatheredCsr) against the one-pass kernels, us, by the
+# size of x (16 uniform columns per row): float32 2 / 4 / 8 / 16 MiB of x 41 /
+# 96 / 346 / 972 one-pass, 50 / 82 / 151 / 329 gathered; float64 and complex64
+# 4 / 8 / 16 MiB 55 / 188 / 514, 67 / 116 / 276 (complex64 77 / 135 / 317).
+# What counts is the x that neighbouring entries touch: a band of 2^18 columns
+# (2 MiB of an 8 MiB float64 x) 82 one-pass, 115 gathered.  Three launches and
+# the slice loads want entries to spread over, 2 / 4 / 6 / 8 / 12 M of them:
+# float64, 8 MiB of x 24 / 46 / 68 / 90 / 104 one-pass, 33 / 46 / 55 / 67 / 88
+# gathered; float32, 4 MiB 15 / 26 / 38 / 48 / 85 against 32 / 35 / 41 / 53 / 62.
+# Beyond 128 slices of 8-byte values the runs get short, and matrices of few
+# long rows (whose column panels add few row ends) stay on the panels: 100,000
+# rows, 4 M columns, 8 M float64 entries 78 on panels, 90 gathered (1 M rows,
+# stream kernel: 130 against 85).
+_GATHER_MIN_NNZ = 6 << 20
+_GATHER_MIN_NNZ_SMALL_X = 12 << 20
+_GATHER_X_BYTES = {4: 4 << 20, 8: 6 << 20}     # by value size
+_GATHER_SMALL_X_BYTES = 6 << 20
+_GATHER_TOUCHED = {4: 24, 8: 40}               # 128 KiB slices of x an average region (32 KiB of x values) touches
+_GATHER_SHORT_RUNS_X_BYTES = 16 << 20          # 8-byte values: 128 slices
+_GATHER_LONG_ROWS = 64
+
+
+def _spmv_gather_worth(plan, value_bytes, one_shot):
+    """Whether a kept prepared matrix takes the two-phase gather: a function
+    of its plan's counts (GatheredCsr.build), or None when it cannot.  The
+    plan costs three reads of the columns, which an unprepared call would not
+    earn back; FLAGSPARSE_SPMV_PANELS and FLAGSPARSE_SPMV_KERNEL keep their
+    kernels."""
+    if one_shot or os.environ.get("FLAGSPARSE_SPMV_PANELS") is not None or os.environ.get("FLAGSPARSE_SPMV_KERNEL"):
+        return None
+    if plan.kernel not in (_lib.FS_KERNEL_MERGE, _lib.FS_KERNEL_STREAM) or value_bytes not in _GATHER_X_BYTES:
+        return None
+    nnz, x_bytes = int(plan.nnz), int(plan.n_cols) * value_bytes
+    if x_bytes < _GATHER_X_BYTES[value_bytes]:
+        return None
+    if nnz < (_GATHER_MIN_NNZ_SMALL_X if x_bytes < _GATHER_SMALL_X_BYTES else _GATHER_MIN_NNZ):
+        return None
+    if (value_bytes == 8 and x_bytes > _GATHER_SHORT_RUNS_X_BYTES and plan.kernel == _lib.FS_KERNEL_MERGE
+            and nnz > _GATHER_LONG_ROWS * int(plan.n_rows)):
+        return None
+    return lambda regions, touched: touched >= _GATHER_TOUCHED[value_bytes] * regions
 
 
 class PanelledCsr:
@@ -320,6 +375,79 @@ class PanelledCsr:
                 _lib.stream_handle(device),
             ),
             "fs_spmv_csr_panels",
+        )
+
+
+class GatheredCsr:
+    """Plan of the two-phase SpMV (fs_spmv_csr_gather): for every entry the
+    16-bit place of its x within its region and, in column-slice order, its
+    16-bit column number; the values and the row pointer stay the caller's.
+
+    indices: the column numbers, two to an int32 word; indptr: the first quad
+    of every region."""
+
+    __slots__ = ("data", "csr_indptr", "n_cols", "part", "pos", "indices", "place", "slice_q", "indptr", "n_quads",
+                 "max_region_quads", "ws_bytes", "n_panels")
+
+    @classmethod
+    def build(cls, data, indices, indptr, n_rows, n_cols, plan, worth):
+        """The plan, or None when the type or sizes are not taken or
+        `worth(regions, slices touched over all regions)` says no.  One device
+        round trip."""
+        lib = _lib.lib()
+        val_t, nnz, device = _lib.value_code(data.dtype), data.numel(), data.device
+        regions = ctypes.c_int64()
+        n_slices = lib.fs_spmv_gather_slices(val_t, n_rows, n_cols, nnz, regions)
+        if n_slices == 0:
+            return None
+        regions = regions.value
+        part = plan.partition(indptr, int(plan.plan.tile_items))
+        stream = _lib.stream_handle(device)
+        counts = torch.empty((2, regions), dtype=torch.int32, device=device)
+        totals = torch.empty(n_slices, dtype=torch.int32, device=device)
+        ws = _lib.workspace(lib.fs_spmv_gather_plan_bytes(val_t, n_rows, n_cols, nnz), device)
+        args = (val_t, _lib.index_code(indices.dtype), n_rows, n_cols, nnz, _lib.ptr(indices), _lib.ptr(part))
+        _lib.check(
+            lib.fs_spmv_gather_count(*args, _lib.ptr(counts[0]), _lib.ptr(counts[1]), _lib.ptr(totals), _lib.ptr(ws),
+                                     ws.numel(), stream),
+            "fs_spmv_gather_count",
+        )
+        sums = torch.cat([counts.sum(1), counts[0].max().view(1)]).tolist()
+        n_quads, touched, max_quads = (int(v) for v in sums)
+        if not worth(regions, touched):
+            return None
+        self = cls()
+        self.data, self.csr_indptr, self.n_cols, self.part = data, indptr, n_cols, part
+        self.n_panels, self.n_quads, self.max_region_quads = n_slices, n_quads, max_quads
+        self.ws_bytes = lib.fs_spmv_gather_workspace_bytes(val_t, n_rows, nnz, n_quads)
+        self.indptr = torch.zeros(regions + 1, dtype=torch.int32, device=device)
+        torch.cumsum(counts[0], 0, out=self.indptr[1:])
+        self.slice_q = torch.zeros(n_slices + 1, dtype=torch.int32, device=device)
+        torch.cumsum(totals, 0, out=self.slice_q[1:])
+        self.pos = torch.empty(nnz, dtype=torch.int16, device=device)
+        self.indices = torch.empty(2 * n_quads, dtype=torch.int32, device=device)
+        self.place = torch.empty(n_quads, dtype=torch.int32, device=device)
+        _lib.check(
+            lib.fs_spmv_gather_fill(*args, _lib.ptr(ws), _lib.ptr(self.indptr), _lib.ptr(self.pos),
+                                    _lib.ptr(self.indices), _lib.ptr(self.place), stream),
+            "fs_spmv_gather_fill",
+        )
+        return self
+
+    def spmv(self, x, y):
+        # the workspace is the call's own: calls on other streams or threads
+        # may share this plan
+        device = self.data.device
+        ws = _lib.workspace(self.ws_bytes, device)
+        _lib.check(
+            _lib.lib().fs_spmv_csr_gather(
+                _lib.value_code(self.data.dtype), _lib.index_code(self.csr_indptr.dtype), self.csr_indptr.numel() - 1,
+                self.n_cols, self.data.numel(), _lib.ptr(self.data), _lib.ptr(self.csr_indptr), _lib.ptr(x),
+                _lib.ptr(y), _lib.ptr(self.part), _lib.ptr(self.pos), _lib.ptr(self.indices), _lib.ptr(self.place),
+                _lib.ptr(self.slice_q), _lib.ptr(self.indptr), self.n_quads, self.max_region_quads, _lib.ptr(ws),
+                ws.numel(), _lib.stream_handle(device),
+            ),
+            "fs_spmv_csr_gather",
         )
 
 

@@ -210,6 +210,43 @@ int fs_spmv_csr_oneshot(int val_t, int idx_t, int ptr_t, int64_t n_rows, int64_t
                         const void* x, void* y, int32_t* flags, hipStream_t stream);
 
 /*
+ * Two-phase SpMV of a kept prepared matrix whose columns spread over an x
+ * larger than L2 serves well (the launch of spmv_csr.py:679-723): x is
+ * gathered slice by slice from LDS into regions of merge-path tiles, then
+ * every region is walked from LDS.  Same products and sums as the merge-path
+ * fs_spmv_csr.  No counterpart in the reference.
+ *
+ * fs_spmv_gather_slices: column slices (ns) and regions of the plan; 0 when
+ * the type or sizes are not taken (complex128, more than 256 slices of 128 KB
+ * of x, 2^31 rows or entries).  Plan, over the 512-item partition of fs_csr_partition:
+ *   fs_spmv_gather_count: quads (groups of four entries of one slice) and
+ *     touched slices of every region (int32[n_regions] each) and the quads of
+ *     every slice (totals, uint32[ns]); ws (fs_spmv_gather_plan_bytes) holds
+ *     the run starts for
+ *   fs_spmv_gather_fill: pos uint16[nnz], idx uint16[4 * n_quads], place
+ *     uint32[n_quads], from region_q (int32[n_regions + 1], the exclusive sum
+ *     of quads; n_quads its last).
+ * fs_spmv_csr_gather: y = A x with slice_q (uint32[ns + 1], the exclusive sum
+ * of totals), max_region_quads the largest entry of quads, and ws of
+ * fs_spmv_gather_workspace_bytes, used during the call only.
+ */
+int fs_spmv_gather_slices(int val_t, int64_t n_rows, int64_t n_cols, int64_t nnz,
+                          int64_t* n_regions);
+size_t fs_spmv_gather_plan_bytes(int val_t, int64_t n_rows, int64_t n_cols, int64_t nnz);
+int fs_spmv_gather_count(int val_t, int idx_t, int64_t n_rows, int64_t n_cols, int64_t nnz,
+                         const void* cols, const void* part, int32_t* quads, int32_t* touched,
+                         uint32_t* totals, void* ws, size_t ws_bytes, hipStream_t stream);
+int fs_spmv_gather_fill(int val_t, int idx_t, int64_t n_rows, int64_t n_cols, int64_t nnz,
+                        const void* cols, const void* part, const void* ws, const int32_t* region_q,
+                        void* pos, void* idx, void* place, hipStream_t stream);
+size_t fs_spmv_gather_workspace_bytes(int val_t, int64_t n_rows, int64_t nnz, int64_t n_quads);
+int fs_spmv_csr_gather(int val_t, int ptr_t, int64_t n_rows, int64_t n_cols, int64_t nnz,
+                       const void* vals, const void* indptr, const void* x, void* y,
+                       const void* part, const void* pos, const void* idx, const void* place,
+                       const void* slice_q, const void* region_q, int64_t n_quads,
+                       int64_t max_region_quads, void* ws, size_t ws_bytes, hipStream_t stream);
+
+/*
  * y = A^T x (conj: A^H x) of a CSR matrix without its transpose, and y += a x
  * over COO entries in any order, by scattered products: every product goes
  * to the bucket of its output (2^k consecutive outputs), then each bucket is
