@@ -72,6 +72,7 @@ EXPORTED_SYMBOLS = (
     "fs_spmv_csr_opt",
     "fs_spmm_workspace_bytes",
     "fs_spmm_tile_items",
+    "fs_spmm_tile_items_sized",
     "fs_spmm_csr",
     "fs_spmm_csr_strided",
     "fs_csr_transpose_workspace_bytes",
@@ -179,6 +180,8 @@ def _declare(lib):
                                     ctypes.POINTER(_i64), _vp]
     lib.fs_spmm_workspace_bytes.restype = _sz
     lib.fs_spmm_workspace_bytes.argtypes = [_i32, _i64, _i64]
+    lib.fs_spmm_tile_items_sized.restype = _i32
+    lib.fs_spmm_tile_items_sized.argtypes = [_i32, _i64, _i64, _i64]
     lib.fs_spmm_tile_items.restype = _i32
     lib.fs_spmm_tile_items.argtypes = [_i32, _i64]
     lib.fs_spmm_csr.restype = _i32

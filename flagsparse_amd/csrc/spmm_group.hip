@@ -354,6 +354,7 @@ inline int group_lpr(int val_t, int64_t n_dense) {
 // Items per sub-tile: a wave covers kGroupWaveItems items whatever its
 // group count (FLAGSPARSE_SPMM_WAVE_ITEMS overrides, 256..16384).
 constexpr int kGroupWaveItems = 2048;
+constexpr int64_t kGroupSkewNnz = 1 << 20;  // from here on a caller may find skewed columns (merge kernel, 512 items)
 inline int group_sub_items(int val_t, int64_t n_dense) {
   int wave_items = kGroupWaveItems;
   if (const char* e = std::getenv("FLAGSPARSE_SPMM_WAVE_ITEMS")) {
@@ -389,6 +390,28 @@ inline int spmm_tile_items_for(int val_t, int64_t n_dense) {
   const int f = forced_kernel();
   if (f == 1 || (f == 0 && wide_rows(val_t, n_dense))) return kMergeTileItems;
   return group_sub_items(val_t, n_dense);
+}
+
+// Items per sub-tile for a matrix of this size: the size above, halved while
+// the matrix gives fewer waves than fill the chip (a group walks its sub-tile
+// one entry after another, so a small matrix in 2048-item waves is a serial
+// chain on a few CUs), down to 128 items per wave.  Measured (us per prepared
+// call, 2048 items always / at least 1024 / 2048 / 4096 / 8192 waves): 2000
+// rows of 9, f32, N = 17: 106 / 24 / 20 / 21 / 21; 100,000 of 16, f32, N = 8:
+// 75 / 45 / 37 / 39 / 50, N = 64 118 / 69 / 85 / 75 / 75; 300,000 of 20, f32,
+// N = 32: 128 / 128 / 128 / 137 / 149, f64, N = 32: 295 / 295 / 295 / 280 /
+// 253.  Smaller sub-tiles cost row fragments, more for narrow B rows: at least
+// 2048 waves there, 4096 with 32 lanes or more per row.
+constexpr int kGroupMinWaveItems = 128;
+inline int spmm_tile_items_sized(int val_t, int64_t n_dense, int64_t n_rows, int64_t nnz) {
+  const int base = spmm_tile_items_for(val_t, n_dense);
+  if (forced_kernel() != 0 || std::getenv("FLAGSPARSE_SPMM_WAVE_ITEMS")) return base;
+  if (wide_rows(val_t, n_dense) && nnz >= kGroupSkewNnz) return base;
+  const int lpr = group_lpr(val_t, n_dense);
+  const int64_t fill = lpr >= 32 ? 4096 : 2048;
+  int wave_items = base * 64 / lpr;
+  while (wave_items > kGroupMinWaveItems && ceil_div(n_rows + nnz, (int64_t)wave_items) < fill) wave_items >>= 1;
+  return wave_items * lpr / 64;
 }
 
 template <class V, int LPR, class T>
@@ -481,6 +504,11 @@ extern "C" int fs_spmm_tile_items(int val_t, int64_t n_dense) {
   return spmm_tile_items_for(val_t, n_dense);
 }
 
+extern "C" int fs_spmm_tile_items_sized(int val_t, int64_t n_dense, int64_t n_rows, int64_t nnz) {
+  if (val_t < FS_F32 || val_t > FS_C128) return kMergeTileItems;
+  return spmm_tile_items_sized(val_t, n_dense, n_rows, nnz);
+}
+
 extern "C" size_t fs_spmm_workspace_bytes(int val_t, int64_t n_tiles, int64_t n_dense) {
   const size_t acc = (val_t == FS_C64 || val_t == FS_C128) ? sizeof(c64) : sizeof(double);
   return (size_t)n_tiles * (size_t)n_dense * 2 * acc;
@@ -497,8 +525,9 @@ extern "C" int fs_spmm_csr_strided(const fs_csr_plan* plan, const void* vals, co
   const int forced = forced_kernel();
   const bool merge = forced == 1 || (forced == 0 && wide_rows(plan->val_t, n_dense) && plan->spmm_wg_cap > 0);
   const bool group = !merge || sbn != 1 || scn != 1;
-  const int want_items = fs_spmm_tile_items(plan->val_t, n_dense);
-  if (tile_items != want_items) return fail(FS_E_INVALID, "fs_spmm_csr: tile_items must come from fs_spmm_tile_items");
+  if (tile_items != fs_spmm_tile_items(plan->val_t, n_dense) &&
+      (!group || tile_items != spmm_tile_items_sized(plan->val_t, n_dense, plan->n_rows, plan->nnz)))
+    return fail(FS_E_INVALID, "fs_spmm_csr: tile_items must come from fs_spmm_tile_items");
   if (n_tiles != ceil_div(plan->n_rows + plan->nnz, tile_items))
     return fail(FS_E_INVALID, "fs_spmm_csr: n_tiles does not match the matrix");
   // C must not overlap itself: distinct (row, column) pairs map to distinct elements.

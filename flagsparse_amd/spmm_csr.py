@@ -307,7 +307,9 @@ class _SpmmPlan:
     def tiling(self, value_dtype, n_dense):
         """(tile_items, n_tiles, partition) of the kernel fs_spmm_csr runs for
         this value type and dense width."""
-        tile_items = int(_lib.lib().fs_spmm_tile_items(_lib.value_code(_compute_dtype(value_dtype)), int(n_dense)))
+        p = self.csr.plan
+        tile_items = int(_lib.lib().fs_spmm_tile_items_sized(_lib.value_code(_compute_dtype(value_dtype)),
+                                                             int(n_dense), p.n_rows, p.nnz))
         return tile_items, self.csr.n_tiles(tile_items), self.csr.partition(self.indptr, tile_items)
 
     def launch_indices(self, indices, value_dtype, n_dense=None):
@@ -450,8 +452,9 @@ def flagsparse_spmm_csr(
     # that the reference raises after its check.
     transposes = _spmm_op_transposes(op_code)
     defer = transposes and out is None and not do_timing and max_segments is None
+    # (row statistics are read for an explicit max_segments only)
     data, indices, indptr, n_rows, n_cols, csr0 = _prepare_spmm_csr_matrix(
-        data, indices, indptr, shape, analyze=not transposes, defer=defer)
+        data, indices, indptr, shape, analyze=not transposes and max_segments is not None, defer=defer)
     pending = csr0 if isinstance(csr0, _PendingCheck) else None
     if pending is not None:
         csr0 = None
@@ -499,8 +502,8 @@ def flagsparse_spmm_csr(
     plan = None
     if n_rows > 0:
         if csr0 is None and max_segments is None:
-            # A^T / A^H: no launch decision needs its row statistics (only an
-            # explicit max_segments does), so no analysis round trip
+            # no launch decision needs the row statistics (only an explicit
+            # max_segments does), so no analysis round trip
             csr0 = CsrPlan.from_sizes(data, indices, indptr, n_rows, n_cols)
         plan = _SpmmPlan(data, indices, indptr, n_rows, n_cols, csr=csr0)
         _check_segment_override(plan.csr.max_row_nnz if max_segments is not None else 0, block_nnz, max_segments)

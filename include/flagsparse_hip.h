@@ -335,6 +335,10 @@ int fs_spmv_csr_opt(int val_t, int idx_t, int ptr_t, int64_t n_rows,
  */
 size_t fs_spmm_workspace_bytes(int val_t, int64_t n_tiles, int64_t n_dense);
 int fs_spmm_tile_items(int val_t, int64_t n_dense);
+
+/* The same for a matrix of this size: smaller sub-tiles where the ones above
+ * would leave the chip idle.  fs_spmm_csr(_strided) takes either size. */
+int fs_spmm_tile_items_sized(int val_t, int64_t n_dense, int64_t n_rows, int64_t nnz);
 int fs_spmm_csr(const fs_csr_plan* plan, const void* vals, const void* cols,
                 const void* indptr, const void* B, int64_t ldb, void* C,
                 int64_t ldc, int64_t n_dense, const void* part_dev,

@@ -1,0 +1,63 @@
+"""The lane-group SpMM on matrices too small for 2048-item waves
+(fs_spmm_tile_items_sized): sub-tiles down to 128 items a wave, rows crossing
+many of them, against the CPU oracle."""
+
+import numpy as np
+import pytest
+import torch
+
+import flagsparse_amd as fs
+from flagsparse_amd import _lib
+from flagsparse_amd import synthetic as S
+from oracle import csr_oracle as O
+from tests._helpers import REL_TOL, VALUE_DTYPES, VALUE_IDS, np_, rel_err
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("n", [1, 4, 17, 32, 64, 130, 256])
+@pytest.mark.parametrize("rows,long_rows", [(3, ()), (40, ((3, 1900),)), (1501, ((0, 2000), (900, 1999), (1500, 700)))])
+@pytest.mark.parametrize("dtype", VALUE_DTYPES, ids=VALUE_IDS)
+def test_small_matrices(dtype, rows, long_rows, n):
+    d, i, p, sh = S.random_csr(rows, 2003, 0.004, dtype, torch.int32, DEV, seed=rows + n, empty_row_every=5,
+                               long_rows=long_rows)
+    B = S.dense(2003, n, dtype, DEV, 3)
+    ref = O.spmm_csr_wide(np_(d), np_(i), np_(p), np_(B), sh)
+    C = fs.flagsparse_spmm_csr(d, i, p, B, sh)
+    assert _lib.last_kernel() == "spmm_group_kernel"
+    assert rel_err(np_(C), ref) <= REL_TOL[dtype]
+    Ct = fs.flagsparse_spmm_csr_run(fs.prepare_spmm_csr_route(d, i, p, sh), B)
+    assert torch.equal(torch.view_as_real(C) if C.is_complex() else C, torch.view_as_real(Ct) if C.is_complex() else Ct)
+
+
+def test_sizes_shrink_with_the_matrix_only():
+    lib = _lib.lib()
+    for n in (1, 32, 64, 128, 256):
+        full = lib.fs_spmm_tile_items(_lib.FS_F32, n)
+        sizes = [lib.fs_spmm_tile_items_sized(_lib.FS_F32, n, 10, nnz) for nnz in (10, 10**5, 10**6, 10**7, 10**8)]
+        assert sizes == sorted(sizes) and sizes[-1] == full and sizes[0] < full
+    # B rows of 512 bytes and more: one size for both kernels once skewed columns are looked for
+    assert lib.fs_spmm_tile_items_sized(_lib.FS_F32, 128, 10, (1 << 20) - 1) < 512
+    assert lib.fs_spmm_tile_items_sized(_lib.FS_F32, 128, 10, 1 << 20) == 512
+
+
+def test_either_tile_size_is_taken():
+    """A caller that sizes its partition by fs_spmm_tile_items is served as before."""
+    d, i, p, sh = S.random_csr(500, 400, 0.03, torch.float32, torch.int32, DEV, seed=2)
+    B = S.dense(400, 40, torch.float32, DEV, 3)
+    route = fs.prepare_spmm_csr_route(d, i, p, sh)
+    plan = route.hip_plan().csr
+    lib = _lib.lib()
+    for items in (lib.fs_spmm_tile_items(_lib.FS_F32, 40), lib.fs_spmm_tile_items_sized(_lib.FS_F32, 40, 500, d.numel())):
+        part, tiles = plan.partition(p, items), plan.n_tiles(items)
+        ws = _lib.workspace(lib.fs_spmm_workspace_bytes(_lib.FS_F32, tiles, 40), B.device)
+        C = torch.empty(500, 40, device=DEV)
+        _lib.check(lib.fs_spmm_csr(plan.plan, _lib.ptr(d), _lib.ptr(i), _lib.ptr(p), _lib.ptr(B), 40, _lib.ptr(C), 40,
+                                   40, _lib.ptr(part), items, tiles, _lib.ptr(ws), ws.numel(),
+                                   _lib.stream_handle(B.device)), "fs_spmm_csr")
+        ref = O.spmm_csr_wide(np_(d), np_(i), np_(p), np_(B), sh)
+        assert rel_err(np_(C), ref) <= REL_TOL[torch.float32]
+    assert lib.fs_spmm_csr(plan.plan, _lib.ptr(d), _lib.ptr(i), _lib.ptr(p), _lib.ptr(B), 40, _lib.ptr(C), 40, 40,
+                           _lib.ptr(part), 96, plan.n_tiles(96), _lib.ptr(ws), ws.numel(),
+                           _lib.stream_handle(B.device)) == _lib.FS_E_INVALID
