@@ -16,7 +16,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libflagsparse_hip.so")
 
-FS_F32, FS_F64, FS_C64, FS_C128 = 0, 1, 2, 3
+FS_F32, FS_F64, FS_C64, FS_C128, FS_F16, FS_BF16 = 0, 1, 2, 3, 4, 5
 FS_I32, FS_I64 = 0, 1
 FS_KERNEL_VECTOR, FS_KERNEL_MERGE, FS_KERNEL_STREAM, FS_KERNEL_NNZBLOCK = 0, 1, 2, 3
 FS_HIST_BINS = 24
@@ -28,6 +28,8 @@ VALUE_TYPE_CODES = {
     torch.complex64: FS_C64,
     torch.complex128: FS_C128,
 }
+# types that the SpMM entry points take besides
+SPMM_HALF_CODES = {torch.float16: FS_F16, torch.bfloat16: FS_BF16}
 INDEX_TYPE_CODES = {torch.int32: FS_I32, torch.int64: FS_I64}
 KERNEL_NAMES = {
     FS_KERNEL_VECTOR: "vector",
@@ -342,6 +344,12 @@ def value_code(dtype):
         return VALUE_TYPE_CODES[dtype]
     except KeyError:
         raise TypeError(f"unsupported value dtype for the HIP kernels: {dtype}") from None
+
+
+def spmm_value_code(dtype):
+    """value_code, with the 16-bit types that the SpMM kernels read as they are."""
+    code = SPMM_HALF_CODES.get(dtype)
+    return value_code(dtype) if code is None else code
 
 
 def index_code(dtype):

@@ -293,10 +293,12 @@ class _SpmmPlan:
         if mode == "0":
             return None
         p = self.csr.plan
+        cdt = _compute_dtype(data.dtype)
         locality = 1.0 if mode == "1" else _spmv_sell_locality(
-            p, indices, self.indptr, False, _sell_codes_possible(data.element_size()))
+            p, indices, self.indptr, False, _sell_codes_possible(torch.empty(0, dtype=cdt).element_size()))
         if locality is not None:
             try:
+                data = data if data.dtype == cdt else data.to(cdt)
                 self._sell = _build_sell(data, indices, self.indptr, int(p.n_rows), int(p.n_cols), int(p.nnz),
                                          locality, force=mode == "1")
             except torch.OutOfMemoryError:
@@ -308,8 +310,8 @@ class _SpmmPlan:
         """(tile_items, n_tiles, partition) of the kernel fs_spmm_csr runs for
         this value type and dense width."""
         p = self.csr.plan
-        tile_items = int(_lib.lib().fs_spmm_tile_items_sized(_lib.value_code(_compute_dtype(value_dtype)),
-                                                             int(n_dense), p.n_rows, p.nnz))
+        tile_items = int(_lib.lib().fs_spmm_tile_items_sized(_lib.spmm_value_code(value_dtype), int(n_dense),
+                                                             p.n_rows, p.nnz))
         return tile_items, self.csr.n_tiles(tile_items), self.csr.partition(self.indptr, tile_items)
 
     def launch_indices(self, indices, value_dtype, n_dense=None):
@@ -324,7 +326,16 @@ class _SpmmPlan:
         kernel (narrower B) runs as fast on int32 indices (N = 32: 0.73 /
         0.74 ms), so those launches skip the widening pass (0.1 ms on 32 M
         entries, which a per-call plan would pay every call).
-        FLAGSPARSE_SPMM_WIDEN_C64=0 never widens (A/B)."""
+        FLAGSPARSE_SPMM_WIDEN_C64=0 never widens (A/B).
+
+        16-bit values: the plan with their type code (the analysis' plan names
+        the type they are widened to)."""
+        half = _lib.SPMM_HALF_CODES.get(value_dtype)
+        if half is not None:
+            half_plan = _lib.FsCsrPlan()
+            ctypes.memmove(ctypes.byref(half_plan), ctypes.byref(self.csr.plan), ctypes.sizeof(half_plan))
+            half_plan.val_t = half
+            return indices, half_plan
         narrow_b = n_dense is not None and n_dense * 8 < 512
         if (value_dtype != torch.complex64 or indices.dtype != torch.int32 or narrow_b
                 or os.environ.get("FLAGSPARSE_SPMM_WIDEN_C64", "1") == "0"):
@@ -343,6 +354,8 @@ class _SpmmPlan:
         512 bytes: for those, fs_spmm_csr picks its kernel by column skew (the
         merge-path kernel, under this residency cap, on skewed columns).
         Narrower launches never read it, so they skip the column count."""
+        if value_dtype in _lib.SPMM_HALF_CODES:
+            return  # the lane-group kernel always
         if self._skew_checked or n_dense * torch.empty(0, dtype=value_dtype).element_size() < 512:
             return
         self._skew_checked = True
@@ -354,6 +367,14 @@ class _SpmmPlan:
             self.csr.plan.spmm_wg_cap = _SPMM_SKEW_WG_CAP
 
 
+def _half_slices(B, C, n_dense):
+    """Whether 16-bit B and C are rows of whole, aligned 8- or 16-byte slices
+    (a C still to be allocated is)."""
+    size = 16 if n_dense % 8 == 0 else 8
+    return n_dense % 4 == 0 and all(
+        t is None or (t.stride(1) == 1 and t.stride(0) * 2 % size == 0 and t.data_ptr() % size == 0) for t in (B, C))
+
+
 def _hip_spmm(data, indices, indptr, B, n_rows, plan, out_dtype, C=None):
     """C = A @ B for a dense B of any non-negative strides (row-major,
     column-major or strided views); returns C.
@@ -363,8 +384,21 @@ def _hip_spmm(data, indices, indptr, B, n_rows, plan, out_dtype, C=None):
     of B or C is made for column-major layouts."""
     device = data.device
     n_dense = int(B.shape[1])
-    cdt = _compute_dtype(data.dtype)
-    data_c = data if data.dtype == cdt else data.to(cdt)
+    # 16-bit values go to the kernel as they are, except wide B that it would
+    # read element by element (widths not multiples of 4, column-major or
+    # unaligned: bfloat16 N = 101, 490 us converted, 690 not) and matrices with
+    # a SELL-64 copy (stencils), which holds float32 values
+    cdt = data.dtype
+    if cdt in _lib.SPMM_HALF_CODES and n_dense > 64 and not _half_slices(B, C, n_dense):
+        cdt = torch.float32
+    sell = None
+    if plan is not None and plan.kept and data.numel() > 0 and n_dense > 0:
+        sell = plan.sell_copy(data, indices)
+        if sell is not None and cdt != sell.vals.dtype:
+            if n_dense % (16 // sell.vals.element_size()) == 0 and B.is_contiguous():
+                cdt = sell.vals.dtype
+            else:
+                sell = None
     B_c = B if B.dtype == cdt else B.to(cdt)
     if any(st < 0 for st in B_c.stride()):
         B_c = B_c.contiguous()
@@ -374,17 +408,17 @@ def _hip_spmm(data, indices, indptr, B, n_rows, plan, out_dtype, C=None):
         C_k = C
     if n_rows == 0 or n_dense == 0:
         return C_k if cdt == out_dtype else C_k.to(out_dtype)
-    sell = plan.sell_copy(data_c, indices) if data.numel() > 0 else None
     if sell is not None and sell.spmm_fits(B_c, C_k):
         sell.spmm(B_c, C_k)
     elif data.numel() == 0:
         C_k.zero_()
     else:
+        data_c = data if data.dtype == cdt else data.to(cdt)
         plan.set_residency(indices, int(plan.csr.plan.n_cols), n_dense, cdt)
         launch_indices, launch_plan = plan.launch_indices(indices, cdt, n_dense)
         tile_items, n_tiles, part = plan.tiling(cdt, n_dense)
         lib = _lib.lib()
-        ws = _lib.workspace(lib.fs_spmm_workspace_bytes(_lib.value_code(cdt), n_tiles, n_dense), device)
+        ws = _lib.workspace(lib.fs_spmm_workspace_bytes(_lib.spmm_value_code(cdt), n_tiles, n_dense), device)
         _lib.check(
             lib.fs_spmm_csr_strided(
                 launch_plan,

@@ -34,9 +34,11 @@
 extern "C" {
 #endif
 
-/* Value types: the reference's SUPPORTED_VALUE_DTYPES minus f16/bf16
- * (sparse_operations/_common.py:21-28). */
-enum fs_value_type { FS_F32 = 0, FS_F64 = 1, FS_C64 = 2, FS_C128 = 3 };
+/* Value types: the reference's SUPPORTED_VALUE_DTYPES
+ * (sparse_operations/_common.py:21-28).  FS_F16 and FS_BF16 are taken by the
+ * SpMM entry points only (fs_spmm_*), for A, B and C alike, with entries and
+ * accumulated in 64 bits. */
+enum fs_value_type { FS_F32 = 0, FS_F64 = 1, FS_C64 = 2, FS_C128 = 3, FS_F16 = 4, FS_BF16 = 5 };
 /* Index types: SUPPORTED_INDEX_DTYPES (_common.py:29). */
 enum fs_index_type { FS_I32 = 0, FS_I64 = 1 };
 /* Column storage of a SELL-64 copy: absolute int32 / int64, the int16
