@@ -81,6 +81,8 @@ EXPORTED_SYMBOLS = (
     "fs_csr_transpose",
     "fs_coo_to_csr_workspace_bytes",
     "fs_coo_to_csr",
+    "fs_coo_to_csr_by_row",
+    "fs_coo_check_ranges",
     "fs_csr_panelize_workspace_bytes",
     "fs_csr_panelize",
     "fs_spmv_panels_workspace_bytes",
@@ -204,6 +206,10 @@ def _declare(lib):
     lib.fs_coo_to_csr_workspace_bytes.argtypes = [_i64, _i64, _i64]
     lib.fs_coo_to_csr.restype = _i32
     lib.fs_coo_to_csr.argtypes = [_i32, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _sz, _vp]
+    lib.fs_coo_to_csr_by_row.restype = _i32
+    lib.fs_coo_to_csr_by_row.argtypes = [_i32, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]
+    lib.fs_coo_check_ranges.restype = _i32
+    lib.fs_coo_check_ranges.argtypes = [_i32, _i64, _i64, _i64, _vp, _vp, _vp, _vp]
     lib.fs_csr_panelize_workspace_bytes.restype = _sz
     lib.fs_csr_panelize_workspace_bytes.argtypes = [_i64, _i64, _i64, _i32]
     lib.fs_csr_panelize.restype = _i32

@@ -832,47 +832,60 @@ __global__ __launch_bounds__(kWgThreads) void wg_count_kernel(const void* __rest
 // the digits); the keys through a digit-sorted LDS copy, out as contiguous
 // runs (or, in the last pass, the column starts to colptr); the payload
 // through the same buffer in windows.
-template <int VW, int MODE>
-__global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel(
-    const void* __restrict__ keys_in, int kind, const typename WgPay<VW>::T* __restrict__ pay_in, int64_t n, int shift,
-    unsigned mask, const uint32_t* __restrict__ offsets, uint32_t* __restrict__ keys_out,
-    typename WgPay<VW>::T* __restrict__ pay_out, WgIO io) {
+// FULL: a whole tile, without lane tests.  (The passes are bound by
+// instruction issue and the barriers between their steps.)
+constexpr int kScatterBufBytes = (int)kWgTile * 8;  // one window of 8-byte payload, two of 12-byte
+static_assert(kScatterBufBytes >= kWgBufBytes, "marks, counters and keys fit");
+template <int VW, int MODE, bool FULL>
+__device__ inline void wg_scatter_tile(const void* __restrict__ keys_in, int kind,
+                                       const typename WgPay<VW>::T* __restrict__ pay_in, int64_t tile, int tcnt,
+                                       int shift, unsigned mask, const uint32_t* __restrict__ offsets,
+                                       uint32_t* __restrict__ keys_out, typename WgPay<VW>::T* __restrict__ pay_out,
+                                       const WgIO& io, uint8_t* s_buf, uint32_t* s_off, int64_t* s_wave) {
   using Pay = typename WgPay<VW>::T;
   constexpr bool kFirst = MODE == kScatterFirst || MODE == kScatterOnly;
   constexpr bool kLast = MODE == kScatterLast || MODE == kScatterOnly;
   constexpr int kWords = kWgMaxDigits / 2;  // counter words per wave
-  __shared__ __attribute__((aligned(16))) uint8_t s_buf[kWgBufBytes];
-  __shared__ uint32_t s_off[kWgMaxDigits];
-  __shared__ int64_t s_wave[kWgWaves];
   const int nd = (int)mask + 1;
   const int t = threadIdx.x;
   const int lane = t & 63;
-  const int w = t >> 6;
-  const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);  // per-XCD tile ranges
-  const int64_t tbase = tile * kWgTile;
-  const int tcnt = n - tbase < kWgTile ? (int)(n - tbase) : (int)kWgTile;
-  const int64_t base = tbase + (int64_t)w * kWgSub;
-  const int cnt = n - base >= kWgSub ? (int)kWgSub : (n - base > 0 ? (int)(n - base) : 0);
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);  // scalar: so are the wave's base addresses
+  const int64_t base = tile * kWgTile + (int64_t)w * kWgSub;
+  const int left = tcnt - w * (int)kWgSub;
+  const int cnt = FULL ? (int)kWgSub : (left < 0 ? 0 : (left < (int)kWgSub ? left : (int)kWgSub));
+  // thread t owns digits [t q, t q + q), q even (both halves of a counter word)
+  constexpr int kQMax = 2 * ((kWgMaxDigits + 2 * kWgThreads - 1) / (2 * kWgThreads));
+  const int q = nd > 2 * kWgThreads ? kQMax : 2;
+  const int d0 = t * q;
   uint32_t key[kWgChunks];
   Pay pay[kWgChunks];
-  wg_load_keys(keys_in, kind, base, cnt, lane, key);
+  wg_load_keys<FULL>(keys_in, kind, base, cnt, lane, key);
+  // digit offsets, loaded before they are needed (a first pass with 12-byte
+  // payload has no registers left for them then)
+  constexpr bool kEarly = !(kFirst && VW == 2);
+  uint32_t off[kQMax];
+  auto load_offsets = [&]() {
+#pragma unroll
+    for (int j = 0; j < kQMax; ++j) off[j] = j < q && d0 + j < nd ? offsets[tile * nd + d0 + j] : 0u;
+  };
+  if constexpr (kEarly) load_offsets();
   if constexpr (kFirst) {
     if constexpr (VW == 1) {
       const uint32_t* vp = static_cast<const uint32_t*>(io.vals) + base + lane;
 #pragma unroll
-      for (int ch = 0; ch < kWgChunks; ++ch) pay[ch] = (uint64_t)(ch * 64 + lane < cnt ? vp[ch * 64] : 0u);
+      for (int ch = 0; ch < kWgChunks; ++ch) pay[ch] = (uint64_t)(FULL || ch * 64 + lane < cnt ? vp[ch * 64] : 0u);
     } else {
       const uint2* vp = static_cast<const uint2*>(io.vals) + base + lane;
 #pragma unroll
       for (int ch = 0; ch < kWgChunks; ++ch) {
-        const uint2 v = ch * 64 + lane < cnt ? vp[ch * 64] : make_uint2(0u, 0u);
+        const uint2 v = FULL || ch * 64 + lane < cnt ? vp[ch * 64] : make_uint2(0u, 0u);
         pay[ch].v0 = v.x;
         pay[ch].v1 = v.y;
       }
     }
     uint32_t row[kWgChunks];
     if (io.other) {
-      wg_load_keys(io.other, io.other64 ? 1 : 0, base, cnt, lane, row);
+      wg_load_keys<FULL>(io.other, io.other64 ? 1 : 0, base, cnt, lane, row);
     } else if (cnt > 0) {
       const int64_t sub = tile * kWgWaves + w;
       auto clamp_row = [&](int64_t r) { return r < 0 ? (int64_t)0 : (r >= io.n_rows ? io.n_rows - 1 : r); };
@@ -898,7 +911,7 @@ __global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel
   } else {
     const Pay* pp = pay_in + base + lane;
 #pragma unroll
-    for (int ch = 0; ch < kWgChunks; ++ch) pay[ch] = ch * 64 + lane < cnt ? pp[ch * 64] : Pay{};
+    for (int ch = 0; ch < kWgChunks; ++ch) pay[ch] = FULL || ch * 64 + lane < cnt ? pp[ch * 64] : Pay{};
     if (io.swap) {
 #pragma unroll
       for (int ch = 0; ch < kWgChunks; ++ch) {
@@ -919,27 +932,30 @@ __global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel
   for (int j = lane; j < (nd + 1) / 2; j += 64) my[j] = 0u;
   wave_sync_t();
   unsigned local[kWgChunks];
+  {
+    // (the counter updates of all chunks are issued before the first is waited for)
+    unsigned old[kWgChunks];
 #pragma unroll
-  for (int ch = 0; ch < kWgChunks; ++ch) {
-    const bool valid = ch * 64 + lane < cnt;
-    const uint64_t active = __ballot(valid);
-    const unsigned digit = (key[ch] >> shift) & mask;
-    const uint64_t peers = match_lanes<kWgMaxBits>(digit, active, mask);
-    const int rank = count_below_t(peers);
-    const unsigned half = (digit & 1u) * 16u;
-    unsigned old = 0;
-    if (valid && rank == 0) old = atomicAdd(&my[digit >> 1], (unsigned)__popcll(peers) << half) >> half;
-    const int leader = peers ? (int)__builtin_ctzll(peers) : lane;
-    old = (unsigned)__builtin_amdgcn_ds_bpermute(leader << 2, (int)(old & 0xffffu));
-    local[ch] = old + (unsigned)rank;
+    for (int ch = 0; ch < kWgChunks; ++ch) {
+      const bool valid = FULL || ch * 64 + lane < cnt;
+      const unsigned digit = (key[ch] >> shift) & mask;
+      const uint64_t peers = match_lanes<kWgMaxBits>(digit, FULL ? ~0ull : __ballot(valid), mask);
+      const int rank = count_below_t(peers);
+      const unsigned half = (digit & 1u) * 16u;
+      old[ch] = 0u;
+      if (valid && rank == 0) old[ch] = atomicAdd(&my[digit >> 1], (unsigned)__popcll(peers) << half) >> half;
+      const int leader = FULL || peers ? (int)__builtin_ctzll(peers) : lane;
+      local[ch] = (unsigned)rank | (unsigned)leader << 8;
+    }
+#pragma unroll
+    for (int ch = 0; ch < kWgChunks; ++ch) {
+      const unsigned o = (unsigned)__builtin_amdgcn_ds_bpermute((int)(local[ch] >> 8) << 2, (int)old[ch]);
+      local[ch] = (o & 0xffffu) + (local[ch] & 0xffu);
+    }
   }
   __syncthreads();
-  // per digit pair: wave bases, then the tile's digit starts (thread t owns
-  // digits [t q, t q + q), q even, so both halves of a counter word)
+  // per digit pair: wave bases, then the tile's digit starts
   {
-    const int q = nd > 2 * kWgThreads ? 2 * ((nd + 2 * kWgThreads - 1) / (2 * kWgThreads)) : 2;
-    const int d0 = t * q;
-    constexpr int kQMax = 2 * ((kWgMaxDigits + 2 * kWgThreads - 1) / (2 * kWgThreads));
     uint32_t sums[kQMax];
     int64_t mine = 0;
 #pragma unroll
@@ -948,17 +964,20 @@ __global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel
       const int d = d0 + j;
       if (j < q && d < nd) {
         uint32_t pre = 0u;  // two 16-bit prefixes
+        uint32_t c[kWgWaves];
+#pragma unroll
+        for (int v = 0; v < kWgWaves; ++v) c[v] = wc[v * kWords + (d >> 1)];
 #pragma unroll
         for (int v = 0; v < kWgWaves; ++v) {
-          const uint32_t c = wc[v * kWords + (d >> 1)];
           wc[v * kWords + (d >> 1)] = pre;
-          pre += c;
+          pre += c[v];
         }
         sums[j] = pre & 0xffffu;
         sums[j + 1] = pre >> 16;
         mine += sums[j] + sums[j + 1];
       }
     }
+    if constexpr (!kEarly) load_offsets();
     int64_t all;
     uint32_t run = (uint32_t)block_exclusive_scan(mine, s_wave, all);
 #pragma unroll
@@ -969,8 +988,8 @@ __global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel
         const uint32_t add = st0 | (st1 << 16);  // starts < kWgTile < 2^16
 #pragma unroll
         for (int v = 0; v < kWgWaves; ++v) wc[v * kWords + (d >> 1)] += add;
-        s_off[d] = offsets[tile * nd + d] - st0;
-        if (d + 1 < nd) s_off[d + 1] = offsets[tile * nd + d + 1] - st1;
+        s_off[d] = off[j] - st0;
+        if (d + 1 < nd) s_off[d + 1] = off[j + 1] - st1;
         run += sums[j] + sums[j + 1];
       }
     }
@@ -988,16 +1007,16 @@ __global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel
   uint32_t* s_key = reinterpret_cast<uint32_t*>(s_buf);
 #pragma unroll
   for (int ch = 0; ch < kWgChunks; ++ch)
-    if (ch * 64 + lane < cnt) s_key[local[ch]] = key[ch];
+    if (FULL || ch * 64 + lane < cnt) s_key[local[ch]] = key[ch];
   __syncthreads();
   static_assert(kWgTile == (int64_t)kWgChunks * kWgThreads, "one sorted position per thread and chunk");
   uint32_t dst[kWgChunks];
 #pragma unroll
   for (int ch = 0; ch < kWgChunks; ++ch) {
     const int i = t + ch * kWgThreads;
-    const uint32_t k = i < tcnt ? s_key[i] : 0u;
+    const uint32_t k = FULL || i < tcnt ? s_key[i] : 0u;
     dst[ch] = s_off[(k >> shift) & mask] + (uint32_t)i;
-    if (i < tcnt) {
+    if (FULL || i < tcnt) {
       if (!kLast || io.colptr == nullptr) {
         keys_out[dst[ch]] = k;
       } else if ((i == 0 || s_key[i - 1] != k) && (int64_t)k < io.n_cols) {
@@ -1015,20 +1034,23 @@ __global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel
   __syncthreads();
   // the payload, in windows of the buffer (each window holds whole rounds
   // of sorted positions, so a thread's positions stay its own)
-  constexpr int kWin = kWgBufBytes / (int)sizeof(Pay) / kWgThreads * kWgThreads;
+  constexpr int kRounds = kScatterBufBytes / (int)sizeof(Pay) / kWgThreads;  // rounds per window
+  constexpr int kWin = kRounds * kWgThreads;
   Pay* s_pay = reinterpret_cast<Pay*>(s_buf);
-  for (int w0 = 0; w0 < tcnt; w0 += kWin) {
+#pragma unroll
+  for (int r0 = 0; r0 < kWgChunks; r0 += kRounds) {
+    const int w0 = r0 * kWgThreads;
+    if (!FULL && w0 >= tcnt) break;
 #pragma unroll
     for (int ch = 0; ch < kWgChunks; ++ch) {
       const unsigned j = local[ch] - (unsigned)w0;
-      if (ch * 64 + lane < cnt && j < (unsigned)kWin) s_pay[j] = pay[ch];
+      if ((FULL || ch * 64 + lane < cnt) && (kRounds >= kWgChunks || j < (unsigned)kWin)) s_pay[j] = pay[ch];
     }
     __syncthreads();
-    const int w1 = w0 + kWin < tcnt ? w0 + kWin : tcnt;
 #pragma unroll
-    for (int ch = 0; ch < kWgChunks; ++ch) {
+    for (int ch = r0; ch < (r0 + kRounds < kWgChunks ? r0 + kRounds : kWgChunks); ++ch) {
       const int i = t + ch * kWgThreads;
-      if (i < w0 || i >= w1) continue;
+      if (!FULL && i >= tcnt) continue;
       const Pay v = s_pay[i - w0];
       if constexpr (kLast) {
         uint32_t r;
@@ -1045,8 +1067,33 @@ __global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel
         pay_out[dst[ch]] = v;
       }
     }
-    __syncthreads();
+    if (r0 + kRounds < kWgChunks) __syncthreads();
   }
+}
+
+template <int VW, int MODE>
+__global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel(
+    const void* __restrict__ keys_in, int kind, const typename WgPay<VW>::T* __restrict__ pay_in, int64_t n, int shift,
+    unsigned mask, const uint32_t* __restrict__ offsets, uint32_t* __restrict__ keys_out,
+    typename WgPay<VW>::T* __restrict__ pay_out, WgIO io) {
+  __shared__ __attribute__((aligned(16))) uint8_t s_buf[kScatterBufBytes];
+  __shared__ uint32_t s_off[kWgMaxDigits];
+  __shared__ int64_t s_wave[kWgWaves];
+  const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);  // per-XCD tile ranges
+  const int64_t left = n - tile * kWgTile;
+  // us of the scatters, before (lane tests, digit offsets loaded late, counter
+  // updates one at a time, two windows) and now: R-MAT 2^21 complex64 455 + 361
+  // -> 456 + 273; COO, 16 M float64 entries, 342 -> 274 in the middle passes;
+  // 33.5 M float32 entries 220 + 289 -> 213 + 286.  12-byte payloads are faster
+  // with the lane tests (the last R-MAT pass 273 / 325 us: registers spill
+  // without them).
+  constexpr bool kWhole = VW == 1;
+  if (kWhole && left >= kWgTile)
+    wg_scatter_tile<VW, MODE, kWhole>(keys_in, kind, pay_in, tile, (int)kWgTile, shift, mask, offsets, keys_out, pay_out,
+                                    io, s_buf, s_off, s_wave);
+  else
+    wg_scatter_tile<VW, MODE, false>(keys_in, kind, pay_in, tile, left < kWgTile ? (int)left : (int)kWgTile, shift, mask, offsets, keys_out, pay_out,
+                                     io, s_buf, s_off, s_wave);
 }
 
 // colptr[c] = min(colptr[c], colptr[c + 1], ...): block minima, their
@@ -2152,9 +2199,10 @@ inline bool coo_wg_applies(int val_t, int64_t n_rows, int64_t n_cols, int64_t nn
          !colptr_from_keys();
 }
 
+// by_row: the row passes alone (entries of a row keep their input order).
 int coo_to_csr_wg(char* ws, int val_t, int idx_t, int64_t n_rows, int64_t n_cols, int64_t nnz, const void* vals,
                   const void* rows, const void* cols, void* out_vals, void* out_cols, void* out_indptr,
-                  hipStream_t s) {
+                  hipStream_t s, bool by_row = false) {
   const WgLayout L = make_wg_layout(std::max(n_rows, n_cols), nnz);
   const int vw = val_t == FS_F32 ? 1 : 2;
   const int64_t n_ptr = n_rows + 1;
@@ -2163,11 +2211,11 @@ int coo_to_csr_wg(char* ws, int val_t, int idx_t, int64_t n_rows, int64_t n_cols
   FS_CHECK_LAUNCH("fill_kernel");
   const int idx_kind = idx_t == FS_I32 ? 0 : 1;
   const int col_bits = key_bits(n_cols), row_bits = key_bits(n_rows);
-  const int col_passes = col_bits == 0 ? 0 : wg_passes(col_bits);
+  const int col_passes = by_row || col_bits == 0 ? 0 : wg_passes(col_bits);
   const int row_passes = wg_passes(row_bits);
   const int passes = col_passes + row_passes;
-  // the first pass reads its keys from the columns (or, with one column,
-  // from the rows) and its second index from the other array
+  // the first pass reads its keys from the columns (or, without column
+  // passes, from the rows) and its second index from the other array
   WgIO io{vals, nullptr, 0, nullptr, n_rows, 0, out_vals, out_cols, 0, out_indptr, 1, n_rows, 0u,
           col_passes > 0 ? rows : cols, idx_t == FS_I64 ? 1 : 0, 0};
   uint32_t* counts = reinterpret_cast<uint32_t*>(ws + L.off_counts);
@@ -2262,6 +2310,79 @@ extern "C" int fs_coo_to_csr(int val_t, int idx_t, int64_t n_rows, int64_t n_col
     case FS_C64: return coo_to_csr_idx<c32>(L, w, idx_t, nnz, n_rows, n_cols, vals, rows, cols, assume_sorted, out_vals, out_cols, out_indptr, stream);
     default: return coo_to_csr_idx<c64>(L, w, idx_t, nnz, n_rows, n_cols, vals, rows, cols, assume_sorted, out_vals, out_cols, out_indptr, stream);
   }
+}
+
+extern "C" int fs_coo_to_csr_by_row(int val_t, int idx_t, int64_t n_rows, int64_t n_cols, int64_t nnz,
+                                    const void* vals, const void* rows, const void* cols, void* out_vals,
+                                    void* out_cols, void* out_indptr, void* ws, size_t ws_bytes, hipStream_t stream) {
+  if (!valid_types(val_t, idx_t, FS_I64)) return fail(FS_E_INVALID, "fs_coo_to_csr_by_row: bad type code");
+  if (n_rows <= 0 || n_cols <= 0 || !coo_wg_applies(val_t, n_rows, n_cols, nnz, 0))
+    return fail(FS_E_INVALID, "fs_coo_to_csr_by_row: type or sizes not supported (use fs_coo_to_csr)");
+  if (!vals || !rows || !cols || !out_vals || !out_cols || !out_indptr)
+    return fail(FS_E_INVALID, "fs_coo_to_csr_by_row: null pointer");
+  if (!ws || ws_bytes < make_wg_layout(std::max(n_rows, n_cols), nnz).total)
+    return fail(FS_E_WORKSPACE, "fs_coo_to_csr_by_row: workspace too small");
+  return coo_to_csr_wg(static_cast<char*>(ws), val_t, idx_t, n_rows, n_cols, nnz, vals, rows, cols, out_vals, out_cols,
+                       out_indptr, stream, true);
+}
+
+// Range check of two index arrays: flag k is set when array k has an entry
+// outside [0, n_k).  16-byte loads where an array is aligned.
+template <class I>
+__device__ inline bool any_outside(const I* __restrict__ p, int64_t n, uint64_t limit, int64_t t0, int64_t stride) {
+  constexpr int kVec = (int)(16 / sizeof(I));
+  using L = I __attribute__((ext_vector_type(kVec)));
+  bool bad = false;
+  int64_t done = 0;
+  if (((uintptr_t)p % 16) == 0) {
+    const L* v = reinterpret_cast<const L*>(p);
+    const int64_t nv = n / kVec;
+    constexpr int kAheadV = 4;
+    for (int64_t i0 = t0; i0 < nv; i0 += kAheadV * stride) {
+      L q[kAheadV];
+#pragma unroll
+      for (int u = 0; u < kAheadV; ++u) q[u] = v[i0 + u * stride < nv ? i0 + u * stride : i0];
+#pragma unroll
+      for (int u = 0; u < kAheadV; ++u)
+#pragma unroll
+        for (int j = 0; j < kVec; ++j) bad |= (uint64_t)(int64_t)q[u][j] >= limit;
+    }
+    done = nv * kVec;
+  }
+  for (int64_t i = done + t0; i < n; i += stride) bad |= (uint64_t)(int64_t)p[i] >= limit;
+  return bad;
+}
+
+template <class I>
+__global__ __launch_bounds__(256) void coo_range_kernel(const I* __restrict__ rows, const I* __restrict__ cols,
+                                                        int64_t n, uint64_t n_rows, uint64_t n_cols,
+                                                        int32_t* __restrict__ flags) {
+  const int64_t t0 = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
+  if (any_outside(rows, n, n_rows, t0, stride)) __hip_atomic_store(flags, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (any_outside(cols, n, n_cols, t0, stride))
+    __hip_atomic_store(flags + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+extern "C" int fs_coo_check_ranges(int idx_t, int64_t n_rows, int64_t n_cols, int64_t nnz, const void* rows,
+                                   const void* cols, int32_t* flags, hipStream_t stream) {
+  if (!(idx_t == FS_I32 || idx_t == FS_I64)) return fail(FS_E_INVALID, "fs_coo_check_ranges: bad type code");
+  if (n_rows < 0 || n_cols < 0 || nnz <= 0 || !rows || !cols || !flags)
+    return fail(FS_E_INVALID, "fs_coo_check_ranges: negative size, no entries or null pointer");
+  void* df = nullptr;
+  FS_CHECK_HIP(hipHostGetDevicePointer(&df, flags, 0));
+  flags[0] = flags[1] = 0;
+  const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(nnz, 256 * 8), 2048);
+  if (idx_t == FS_I64)
+    hipLaunchKernelGGL((coo_range_kernel<int64_t>), dim3(blocks), dim3(256), 0, stream,
+                       static_cast<const int64_t*>(rows), static_cast<const int64_t*>(cols), nnz, (uint64_t)n_rows,
+                       (uint64_t)n_cols, static_cast<int32_t*>(df));
+  else
+    hipLaunchKernelGGL((coo_range_kernel<int32_t>), dim3(blocks), dim3(256), 0, stream,
+                       static_cast<const int32_t*>(rows), static_cast<const int32_t*>(cols), nnz, (uint64_t)n_rows,
+                       (uint64_t)n_cols, static_cast<int32_t*>(df));
+  FS_CHECK_LAUNCH("coo_range_kernel");
+  FS_CHECK_HIP(hipStreamSynchronize(stream));
+  return FS_OK;
 }
 
 // Panel layout: the [panel][sub-tile] counts and their scan partials, the

@@ -2,8 +2,8 @@
 
 The reference coalesces duplicate (row, col) entries, lex-sorts them and
 runs a row-run Triton kernel (complex dtypes through an atomic kernel),
-spmm_coo.py:101-142, 417-595.  Here one device radix sort
-(``fs_coo_to_csr``, stable on row * n_cols + col) turns the COO into the
+spmm_coo.py:101-142, 417-595.  Here one device radix sort by row
+(``fs_coo_to_csr_by_row``, stable) turns the COO into the
 CSR the SpMM kernels walk; duplicates stay separate entries of the same
 row, which is the same product up to rounding (the sum distributes), and
 the merge-path SpMM kernel accumulates them in a fixed order (no atomics,
@@ -20,9 +20,12 @@ import time
 
 import torch
 
+from . import _lib
 from ._common import _INDEX_LIMIT_INT32, SUPPORTED_INDEX_DTYPES
+from ._csr import CsrPlan
 from .coo import coo_to_csr_for_spmv
-from .spmm_csr import SUPPORTED_SPMM_VALUE_DTYPES, flagsparse_spmm_csr
+from .spmm_csr import SUPPORTED_SPMM_VALUE_DTYPES, _hip_spmm, _SpmmPlan
+from .spmv_csr import _oneshot_flags
 
 
 def _prepare_spmm_coo_inputs(data, row, col, B, shape):
@@ -56,7 +59,21 @@ def _prepare_spmm_coo_inputs(data, row, col, B, shape):
     if nnz > _INDEX_LIMIT_INT32:
         # same limit and message as the reference's COO kernel contract
         raise ValueError("nnz exceeds the int32 range supported by the Triton COO kernel")
-    if nnz > 0:
+    if nnz > 0 and max(n_rows, n_cols) <= _INDEX_LIMIT_INT32:
+        idx_dtype = torch.promote_types(row.dtype, col.dtype)
+        row, col = row.to(idx_dtype).contiguous(), col.to(idx_dtype).contiguous()
+        flags = _oneshot_flags()
+        _lib.check(
+            _lib.lib().fs_coo_check_ranges(_lib.index_code(idx_dtype), n_rows, n_cols, nnz, _lib.ptr(row), _lib.ptr(col),
+                                           flags.data_ptr(), _lib.stream_handle(data.device)),
+            "fs_coo_check_ranges",
+        )
+        bad_row, bad_col = flags.tolist()[:2]
+        if bad_row:
+            raise IndexError("row indices out of range for n_rows")
+        if bad_col:
+            raise IndexError("col indices out of range for n_cols")
+    elif nnz > 0:
         lo_hi = torch.stack(
             [row.min().to(torch.int64), row.max().to(torch.int64), col.min().to(torch.int64), col.max().to(torch.int64)]
         ).cpu().tolist()
@@ -82,6 +99,31 @@ def _check_out(out, device, n_rows, n_dense, dtype):
         raise ValueError("out shape/dtype must match result")
 
 
+def _rows_together(data, row, col, shape):
+    """CSR of valid COO entries, each row's in their input order: the product
+    needs rows, not sorted columns, so the sort's column passes are left out
+    (two passes instead of four for 2^19 rows and columns) where the type and
+    sizes allow."""
+    n_rows, n_cols = shape
+    nnz = data.numel()
+    if nnz == 0 or data.dtype == torch.complex128 or max(shape) > _INDEX_LIMIT_INT32:
+        return coo_to_csr_for_spmv(data, row, col, shape)
+    lib = _lib.lib()
+    out_data, out_cols = torch.empty_like(data), torch.empty(nnz, dtype=torch.int32, device=data.device)
+    indptr = torch.empty(n_rows + 1, dtype=torch.int64, device=data.device)
+    idx_dtype = torch.promote_types(row.dtype, col.dtype)
+    row, col = row.to(idx_dtype), col.to(idx_dtype)
+    ws = _lib.workspace(lib.fs_coo_to_csr_workspace_bytes(n_rows, n_cols, nnz), data.device)
+    rc = lib.fs_coo_to_csr_by_row(
+        _lib.value_code(data.dtype), _lib.index_code(idx_dtype), n_rows, n_cols, nnz, _lib.ptr(data), _lib.ptr(row),
+        _lib.ptr(col), _lib.ptr(out_data), _lib.ptr(out_cols), _lib.ptr(indptr), _lib.ptr(ws), ws.numel(),
+        _lib.stream_handle(data.device))
+    if rc == _lib.FS_E_INVALID:  # a size the workgroup passes do not take
+        return coo_to_csr_for_spmv(data, row, col, shape)
+    _lib.check(rc, "fs_coo_to_csr_by_row")
+    return out_data, out_cols, indptr
+
+
 def flagsparse_spmm_coo(data, row, col, B, shape, block_n=None, block_nnz=256, out=None, return_time=False):
     """COO SpMM: C = A @ B (spmm_coo.py:696-723).  No op argument, like the
     reference.  Returns C, or (C, ms) with return_time."""
@@ -94,16 +136,15 @@ def flagsparse_spmm_coo(data, row, col, B, shape, block_n=None, block_nnz=256, o
         _check_out(out, data.device, n_rows, n_dense, data.dtype)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
-    idx_dtype = torch.promote_types(row.dtype, col.dtype)
-    # float16 / bfloat16 are sorted and multiplied as float32 (their compute
-    # dtype), and the result is cast back to the input dtype
+    # float16 / bfloat16 values are sorted as float32, which holds them exactly
     half = data.dtype in (torch.float16, torch.bfloat16)
-    data_k = data.to(torch.float32) if half else data
-    B_k = B.to(torch.float32) if half else B
-    d, c32, indptr = coo_to_csr_for_spmv(data_k, row.to(idx_dtype), col.to(idx_dtype), (n_rows, n_cols))
-    C = flagsparse_spmm_csr(d, c32, indptr, B_k, (n_rows, n_cols), block_nnz=block_nnz)
+    d, c32, indptr = _rows_together(data.to(torch.float32) if half else data, row, col, (n_rows, n_cols))
     if half:
-        C = C.to(data.dtype)
+        d = d.to(data.dtype)
+    plan = None
+    if n_rows > 0:
+        plan = _SpmmPlan(d, c32, indptr, n_rows, n_cols, csr=CsrPlan.from_sizes(d, c32, indptr, n_rows, n_cols))
+    C = _hip_spmm(d, c32, indptr, B, n_rows, plan, data.dtype)
     torch.cuda.synchronize()
     elapsed_ms = (time.perf_counter() - t0) * 1000.0
     if out is not None:

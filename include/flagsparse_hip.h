@@ -431,6 +431,25 @@ int fs_coo_to_csr(int val_t, int idx_t, int64_t n_rows, int64_t n_cols,
                   hipStream_t stream);
 
 /*
+ * fs_coo_to_csr with the entries of a row left in their input order (the
+ * column passes are left out): what a product needs of the COO SpMM's sort
+ * (spmm_coo.py:101-142).  4- and 8-byte values, sizes below 2^32; workspace as
+ * fs_coo_to_csr.
+ */
+int fs_coo_to_csr_by_row(int val_t, int idx_t, int64_t n_rows, int64_t n_cols, int64_t nnz,
+                         const void* vals, const void* rows, const void* cols, void* out_vals,
+                         void* out_cols, void* out_indptr, void* ws, size_t ws_bytes,
+                         hipStream_t stream);
+
+/*
+ * Range check of COO indices (spmm_coo.py:372-383): flags[0] / flags[1] (pinned
+ * host memory, zeroed here, valid on return: the call synchronises `stream`)
+ * are set when a row / column lies outside [0, n_rows) / [0, n_cols).
+ */
+int fs_coo_check_ranges(int idx_t, int64_t n_rows, int64_t n_cols, int64_t nnz, const void* rows,
+                        const void* cols, int32_t* flags, hipStream_t stream);
+
+/*
  * Column panels for SpMV on matrices whose x does not fit one XCD's L2.
  * No counterpart call in the reference: it is part of what prepare_spmv_csr
  * (spmv_csr.py:591-676) may precompute once per matrix, and
