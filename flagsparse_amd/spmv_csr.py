@@ -232,6 +232,14 @@ class PreparedCsrSpmv:
                 self._carry = _lib.workspace(p.carry_bytes, data.device)
         return self._plan
 
+    def drop_gather(self):
+        """Leaves the two-phase gather for the one-pass kernel of the plan."""
+        p = self._plan.plan
+        if p.kernel == _lib.FS_KERNEL_MERGE:
+            self._part = self._plan.partition(self.kernel_indptr, int(p.tile_items))
+            self._carry = _lib.workspace(p.carry_bytes, self.data.device)
+        self._panels = None
+
     def compute_data(self):
         """Values in the dtype the kernel runs in (f16/bf16 -> f32, cached)."""
         cdt = _compute_dtype(self.data.dtype)
@@ -1072,7 +1080,17 @@ def _hip_spmv_csr_impl_prepared(prepared, x):
     plan = prepared.hip_plan()
     copy = prepared._sell if prepared._sell is not None else prepared._panels
     if copy is not None:
-        copy.spmv(x_in, y_out)
+        try:
+            copy.spmv(x_in, y_out)
+        except torch.OutOfMemoryError:
+            # a gathered call's workspace is its own: without room for it the
+            # CSR kernels run, from here on
+            if not isinstance(copy, GatheredCsr):
+                raise
+            torch.cuda.empty_cache()
+            prepared.drop_gather()
+            copy = None
+    if copy is not None:
         if y_out is not y:
             y.copy_(y_out)
         return y

@@ -148,3 +148,21 @@ def test_plan_out_of_memory_keeps_the_csr_kernels(any_size, monkeypatch):
     y = fs.flagsparse_spmv_csr(x=x, prepared=fs.prepare_spmv_csr(*mat))
     assert _lib.last_kernel() != "spmv_region_kernel"
     assert torch.allclose(y, want, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("lengths", [[9] * 4000, [5000] + [3] * 3000], ids=["stream", "merge"])
+def test_call_without_room_for_its_workspace(any_size, monkeypatch, lengths):
+    mat = _matrix(lengths, 50000, torch.float32, torch.int32, torch.int32, 8)
+    x = S.vector(50000, torch.float32, DEV, 9)
+    prep = fs.prepare_spmv_csr(*mat)
+    want = fs.flagsparse_spmv_csr(x=x, prepared=prep)
+    assert _lib.last_kernel() == "spmv_region_kernel"
+
+    def no_memory(self, x, y):
+        raise torch.OutOfMemoryError("injected")
+
+    monkeypatch.setattr(spmv_mod.GatheredCsr, "spmv", no_memory)
+    for _ in range(2):
+        y = fs.flagsparse_spmv_csr(x=x, prepared=prep)
+        assert _lib.last_kernel() != "spmv_region_kernel"
+        assert torch.allclose(y, want, rtol=1e-6, atol=1e-6)
