@@ -259,8 +259,8 @@ __device__ inline bool region_tile_loads(const V* __restrict__ vals, const uint1
 }
 
 // Phase 2: one region per workgroup.  A wave's first tile is loaded before the
-// region is waited for, and tile i + 1 before tile i is walked.  It reads at
-// 3.9 TB/s (power-law 4 M float32: 784 MB in 201 us); with lane tests in whole
+// region is waited for, and tile i + 1 before tile i is walked.  It moves
+// 4.1 TB/s (power-law 4 M float32: 822 MB in 201 us); with lane tests in whole
 // tiles it was bound by instruction issue (212 us, SIMDs active 88%).
 template <class V, class P>
 __global__ __launch_bounds__(256) void spmv_region_kernel(const V* __restrict__ vals, const uint16_t* __restrict__ pos,
