@@ -581,7 +581,7 @@ __global__ __launch_bounds__(256) void spmv_stream_t_kernel(
 //     raises the reference's error for any flag and discards y;
 //   - the block's rows go through K3t's LDS stage with 4 lanes per row when
 //     their entries fit it, else as two 32-row halves with 8 lanes per row,
-//     else row by row with the whole workgroup per row (long rows).
+//     else row by row: 16 lanes, a wave or the workgroup by row length.
 // flags[0..3]: start, end, decrease, column (set to 1; zeroed by the host).
 // ---------------------------------------------------------------------------
 // Column range check of the one-shot kernel: column c is in [0, n_cols)
@@ -771,20 +771,51 @@ __global__ __launch_bounds__(256) void spmv_oneshot_kernel(
                                   nc, bad);
       }
     } else {
-      // long rows: the whole workgroup per row, straight from global memory
-      const int lane = t & 63;
-      for (int r = 0; r < rows; ++r) {
-        const int a = s_off[r], b = s_off[r + 1];
+      // An uneven block, straight from global memory: rows of up to 64 entries
+      // by 16 lanes (16 rows at once), up to 4096 by a wave, longer ones by
+      // the workgroup.  (Every row by the whole workgroup, with a barrier and
+      // a dependent load and gather for each of 64 rows: R-MAT 2^20 float64 1488
+      // us a call against 1005, 1 M power-law rows float32 277 against 204.)
+      constexpr int kShort = 64, kMid = 4096;
+      const auto last = ColGuard<I>::last(nc);
+      // entries first, first + stride, ... below len of the row at S + a, N loads in flight
+      auto row_part = [&](auto n_tag, int a, int len, int first, int stride) -> A {
+        constexpr int N = decltype(n_tag)::value;
         A acc = T::zero();
-        for (int q = a + t; q < b; q += 256) {
-          const auto u = (typename ColGuard<I>::U)cols[S + q];
-          const auto last = ColGuard<I>::last(nc);
-          if (u > last) bad = true;
-          acc = T::fma(vals[S + q], x[u < last ? u : last], acc);
-        }
+        for (int q0 = first; q0 - first < len; q0 += N * stride) {
+          V v[N], xv[N];
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) acc = add(acc, shfl(acc, lane ^ off));  // fixed order
-        if (lane == 0) s_red[t >> 6] = acc;
+          for (int k = 0; k < N; ++k) {
+            const int q = q0 + k * stride < len ? q0 + k * stride : len - 1;  // past the end: the last entry, not added
+            const auto u = (typename ColGuard<I>::U)cols[S + a + q];
+            v[k] = vals[S + a + q];
+            if (u > last) bad = true;
+            xv[k] = x[u < last ? u : last];
+          }
+#pragma unroll
+          for (int k = 0; k < N; ++k)
+            if (q0 + k * stride < len) acc = T::fma(v[k], xv[k], acc);
+        }
+        return acc;
+      };
+      const int lane = t & 63, w = t >> 6;
+      for (int r = t >> 4; r < rows; r += 16) {
+        const int a = s_off[r], len = s_off[r + 1] - a;
+        if (len > kShort) continue;
+        const A sum = group_sum<16>(row_part(std::integral_constant<int, 4>{}, a, len, t & 15, 16));
+        if ((t & 15) == 0) y[rb0 + r] = T::out(sum);
+      }
+      for (int r = w; r < rows; r += 4) {
+        const int a = s_off[r], len = s_off[r + 1] - a;
+        if (len <= kShort || len > kMid) continue;
+        const A sum = wave_total(row_part(std::integral_constant<int, 4>{}, a, len, lane, 64));
+        if (lane == 0) y[rb0 + r] = T::out(sum);
+      }
+      for (int r = 0; r < rows; ++r) {
+        const int a = s_off[r], len = s_off[r + 1] - a;
+        if (len <= kMid) continue;  // the same for the whole workgroup
+        const A sum = wave_total(row_part(std::integral_constant<int, 4>{}, a, len, t, 256));
+        if (lane == 0) s_red[w] = sum;
         __syncthreads();
         if (t == 0) y[rb0 + r] = T::out(add(add(s_red[0], s_red[1]), add(s_red[2], s_red[3])));
         __syncthreads();

@@ -1394,19 +1394,23 @@ def _spmv_transposed_oneshot(data, indices, indptr, x, shape, op_code, index_fal
     (up to 2^23 columns, 2^22 for complex128); beyond, the transpose, which
     stays in bounds on any input and runs the structure check in its passes
     (fs_csr_transpose_checked), and the one-launch SpMV on A^T queued behind
-    it.  None when the general path must run: an invalid x, empty shapes,
-    float16 / bfloat16, complex128 beyond the scatter's sizes, a forced
-    kernel or a failed launch."""
+    it.  float16 / bfloat16 run as float32 and are rounded back.  None when
+    the general path must run: an invalid x, empty shapes, complex128 beyond
+    the scatter's sizes, a forced kernel or a failed launch."""
     if os.environ.get("FLAGSPARSE_SPMV_ONESHOT", "1") == "0" or os.environ.get("FLAGSPARSE_SPMV_KERNEL"):
         return None
     data, indices, indptr, n_rows, n_cols = _validate_spmv_host(data, indices, indptr, shape, index_fallback_policy)
     nnz = data.numel()
-    if data.dtype not in HIP_VALUE_DTYPES or n_rows == 0 or n_cols == 0 or nnz == 0:
+    if n_rows == 0 or n_cols == 0 or nnz == 0:
         return None
     try:
         x = _validate_spmv_x_for(x, data.dtype, n_rows, data.device)
     except (TypeError, ValueError):
         return None
+    if data.dtype not in HIP_VALUE_DTYPES:  # float16 / bfloat16: computed in float32 (_compute_dtype)
+        cdt = _compute_dtype(data.dtype)
+        y = _spmv_transposed_oneshot(data.to(cdt), indices, indptr, x.to(cdt), shape, op_code, index_fallback_policy)
+        return None if y is None else y.to(data.dtype)
     lib = _lib.lib()
     ws_bytes = lib.fs_spmv_scatter_workspace_bytes(_lib.value_code(data.dtype), n_cols, nnz)
     if ws_bytes > 0:
@@ -1436,24 +1440,36 @@ def _spmv_transposed_oneshot(data, indices, indptr, x, shape, op_code, index_fal
     return y
 
 
+# float16 / bfloat16 take the one-launch call while a call is what counts (3000
+# rows of 10: 83 us on the general path, 36 in one launch); above, hub rows
+# would cost more than its saved launches (R-MAT 2^20: 226 against 816 us).
+_ONESHOT_HALF_MAX_NNZ = 1 << 18
+
+
 def _spmv_oneshot(data, indices, indptr, x, shape, index_fallback_policy, timed):
     """The unprepared y = A x in one launch (fs_spmv_csr_oneshot): the
     kernel checks the structure while it computes, and the reference's
     errors are raised here, in its order (spmv_csr.py:546-558), before y
     is returned or `out` is written.  Returns (y, compute_ms) or None when
     the general path must run: an invalid x (its error comes after the
-    structure checks), empty shapes, float16 / bfloat16, a forced kernel,
-    or a failed launch (the general path holds the int64 -> int32 fallback)."""
+    structure checks), empty shapes, large float16 / bfloat16, a forced
+    kernel, or a failed launch (the general path holds the int64 -> int32 fallback)."""
     if os.environ.get("FLAGSPARSE_SPMV_ONESHOT", "1") == "0" or os.environ.get("FLAGSPARSE_SPMV_KERNEL"):
         return None
     data, indices, indptr, n_rows, n_cols = _validate_spmv_host(data, indices, indptr, shape, index_fallback_policy)
     nnz = data.numel()
-    if data.dtype not in HIP_VALUE_DTYPES or n_rows == 0 or n_cols == 0 or nnz == 0:
+    if n_rows == 0 or n_cols == 0 or nnz == 0:
         return None
     try:
         x = _validate_spmv_x_for(x, data.dtype, n_cols, data.device)
     except (TypeError, ValueError):
         return None
+    if data.dtype not in HIP_VALUE_DTYPES:  # float16 / bfloat16: computed in float32 (_compute_dtype)
+        if nnz > _ONESHOT_HALF_MAX_NNZ:
+            return None
+        cdt = _compute_dtype(data.dtype)
+        done = _spmv_oneshot(data.to(cdt), indices, indptr, x.to(cdt), shape, index_fallback_policy, timed)
+        return None if done is None else (done[0].to(data.dtype), done[1])
     y = torch.empty(n_rows, dtype=data.dtype, device=data.device)
     flag_t = _oneshot_flags()
     if timed:

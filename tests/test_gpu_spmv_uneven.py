@@ -1,0 +1,53 @@
+"""The one-launch SpMV's uneven 64-row blocks: rows on both sides of 64 and
+4096 entries in one block (16 lanes, a wave, the workgroup), and 16-bit
+values through the same call, against the CPU oracle."""
+
+import numpy as np
+import pytest
+import torch
+
+import flagsparse_amd as fs
+from flagsparse_amd import _lib
+from flagsparse_amd import synthetic as S
+from oracle import csr_oracle as O
+from tests._helpers import INDEX_DTYPES, INDEX_IDS, REL_TOL, VALUE_DTYPES, VALUE_IDS, np_, rel_err
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+LENGTHS = [0, 1, 15, 16, 17, 63, 64, 65, 255, 256, 257, 4095, 4096, 4097, 9000] + [3] * 100 + [5000, 0, 0]
+
+
+def _matrix(dtype, index_dtype, lengths=LENGTHS, n_cols=20011):
+    g = np.random.default_rng(3)
+    ptr = np.concatenate([[0], np.cumsum(lengths)])
+    cols = torch.tensor(g.integers(0, n_cols, ptr[-1]), device=DEV).to(index_dtype)
+    return S.vector(int(ptr[-1]), dtype, DEV, 4), cols, torch.tensor(ptr, device=DEV).to(index_dtype), (len(lengths), n_cols)
+
+
+@pytest.mark.parametrize("index_dtype", INDEX_DTYPES, ids=INDEX_IDS)
+@pytest.mark.parametrize("dtype", VALUE_DTYPES, ids=VALUE_IDS)
+def test_row_lengths(dtype, index_dtype):
+    d, i, p, sh = _matrix(dtype, index_dtype)
+    x = S.vector(sh[1], dtype, DEV, 5)
+    y = fs.flagsparse_spmv_csr(d, i, p, x, sh)
+    assert _lib.last_kernel() == "spmv_oneshot_kernel"
+    assert rel_err(np_(y), O.spmv_csr_wide(np_(d), np_(i), np_(p), np_(x), sh)) <= REL_TOL[dtype]
+    assert torch.equal(torch.view_as_real(y) if y.is_complex() else y,
+                       (lambda z: torch.view_as_real(z) if z.is_complex() else z)(fs.flagsparse_spmv_csr(d, i, p, x, sh)))
+    i[int(p[14]) + 4500] = sh[1]  # a stray column in the longest row
+    with pytest.raises(IndexError, match="out of range for n_cols"):
+        fs.flagsparse_spmv_csr(d, i, p, x, sh)
+
+
+@pytest.mark.parametrize("op", ["non", "trans", "conj"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+def test_half_values(dtype, op):
+    d, i, p, sh = _matrix(torch.float32, torch.int32, [7, 0, 70, 300, 2] * 40, 900)
+    d = d.to(dtype)
+    x = S.vector(sh[1] if op == "non" else sh[0], torch.float32, DEV, 5).to(dtype)
+    y = fs.flagsparse_spmv_csr(d, i, p, x, sh, op=op)
+    assert y.dtype == dtype
+    want = fs.flagsparse_spmv_csr(d.float(), i, p, x.float(), sh, op=op).to(dtype)
+    assert torch.equal(y, want)
+    with pytest.raises(TypeError, match="x dtype must match"):
+        fs.flagsparse_spmv_csr(d, i, p, x.float(), sh, op=op)
