@@ -399,9 +399,9 @@ class GatheredCsr:
 
     @classmethod
     def build(cls, data, indices, indptr, n_rows, n_cols, plan, worth):
-        """The plan, or None when the type or sizes are not taken or
-        `worth(regions, slices touched over all regions)` says no.  One device
-        round trip."""
+        """The plan, complete in device memory, or None when the type or sizes
+        are not taken or `worth(regions, slices touched over all regions)` says
+        no.  Two device round trips."""
         lib = _lib.lib()
         val_t, nnz, device = _lib.value_code(data.dtype), data.numel(), data.device
         regions = ctypes.c_int64()
@@ -440,6 +440,9 @@ class GatheredCsr:
                                     _lib.ptr(self.indices), _lib.ptr(self.place), stream),
             "fs_spmv_gather_fill",
         )
+        # calls on other streams store at the places this wrote: without a
+        # wait they could read the arrays before it ran
+        torch.cuda.current_stream(device).synchronize()
         return self
 
     def spmv(self, x, y):
