@@ -395,7 +395,7 @@ class GatheredCsr:
     of every region."""
 
     __slots__ = ("data", "csr_indptr", "n_cols", "part", "pos", "indices", "place", "slice_q", "indptr", "n_quads",
-                 "max_region_quads", "ws_bytes", "n_panels")
+                 "max_region_quads", "ws_bytes", "n_panels", "stream")
 
     @classmethod
     def build(cls, data, indices, indptr, n_rows, n_cols, plan, worth):
@@ -443,12 +443,20 @@ class GatheredCsr:
         # calls on other streams store at the places this wrote: without a
         # wait they could read the arrays before it ran
         torch.cuda.current_stream(device).synchronize()
+        self.stream = stream
         return self
 
     def spmv(self, x, y):
         # the workspace is the call's own: calls on other streams or threads
         # may share this plan
         device = self.data.device
+        stream = _lib.stream_handle(device)
+        if stream != self.stream:
+            # a dropped plan's memory waits for the calls still queued here: its
+            # next owner would overwrite their store places
+            current = torch.cuda.current_stream(device)
+            for t in (self.part, self.pos, self.indices, self.place, self.slice_q, self.indptr):
+                t.record_stream(current)
         ws = _lib.workspace(self.ws_bytes, device)
         _lib.check(
             _lib.lib().fs_spmv_csr_gather(
@@ -456,7 +464,7 @@ class GatheredCsr:
                 self.n_cols, self.data.numel(), _lib.ptr(self.data), _lib.ptr(self.csr_indptr), _lib.ptr(x),
                 _lib.ptr(y), _lib.ptr(self.part), _lib.ptr(self.pos), _lib.ptr(self.indices), _lib.ptr(self.place),
                 _lib.ptr(self.slice_q), _lib.ptr(self.indptr), self.n_quads, self.max_region_quads, _lib.ptr(ws),
-                ws.numel(), _lib.stream_handle(device),
+                ws.numel(), stream,
             ),
             "fs_spmv_csr_gather",
         )

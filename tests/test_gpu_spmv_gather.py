@@ -166,3 +166,25 @@ def test_call_without_room_for_its_workspace(any_size, monkeypatch, lengths):
         y = fs.flagsparse_spmv_csr(x=x, prepared=prep)
         assert _lib.last_kernel() != "spmv_region_kernel"
         assert torch.allclose(y, want, rtol=1e-6, atol=1e-6)
+
+
+def test_replayed_from_a_graph(any_size):
+    g = np.random.default_rng(2)
+    mat = _matrix(g.integers(0, 40, 9000), 70001, torch.float32, torch.int32, torch.int32, 8)
+    x = S.vector(70001, torch.float32, DEV, 9)
+    prep = fs.prepare_spmv_csr(*mat)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        fs.flagsparse_spmv_csr(x=x, prepared=prep)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = fs.flagsparse_spmv_csr(x=x, prepared=prep)
+    for _ in range(3):
+        x.mul_(1.5)
+        want = fs.flagsparse_spmv_csr(x=x, prepared=prep)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)

@@ -40,6 +40,7 @@ def recorded(monkeypatch):
         fs_spmv_gather_workspace_bytes=lambda *a: 256,
         fs_spmv_gather_count=count,
         fs_spmv_gather_fill=lambda *a: events.append("fill") or 0,
+        fs_spmv_csr_gather=lambda *a: events.append(f"call on {a[-1]}") or 0,
     )
     stream = SimpleNamespace(synchronize=lambda: events.append("synchronize"))
     monkeypatch.setattr(_lib, "lib", lambda: lib)
@@ -58,3 +59,28 @@ def test_build_returns_a_finished_plan(recorded):
     plan, events = recorded
     assert plan.n_quads == 6 and plan.max_region_quads == 2
     assert events == ["count", "fill", "synchronize"]
+
+
+def test_a_call_on_another_stream_keeps_the_plan_alive(recorded, monkeypatch):
+    plan, events = recorded
+    x, y = torch.ones(9), torch.empty(1)
+    kept = []
+
+    class Tensor:
+        def __init__(self, t):
+            self.t = t
+
+        def record_stream(self, stream):
+            kept.append(self.t.data_ptr())
+
+        def __getattr__(self, name):
+            return getattr(self.t, name)
+
+    names = ("part", "pos", "indices", "place", "slice_q", "indptr")
+    for name in names:
+        setattr(plan, name, Tensor(getattr(plan, name)))
+    plan.spmv(x, y)
+    assert kept == [] and events[-1] == "call on 11"
+    monkeypatch.setattr(_lib, "stream_handle", lambda device: 12)
+    plan.spmv(x, y)
+    assert kept == [getattr(plan, name).data_ptr() for name in names] and events[-1] == "call on 12"
