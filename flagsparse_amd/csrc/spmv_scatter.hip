@@ -42,6 +42,7 @@
 // with the structure is reported through the flags and the caller discards y.
 #include "fs_common.hpp"
 #include "radix_tile.hpp"
+#include "scatter_segments.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -195,9 +196,8 @@ __global__ __launch_bounds__(kWgThreads) void scatter_count_kernel(const I* __re
   for (int d = t; d < nd; d += kWgThreads) counts[(int64_t)blockIdx.x * nd + d] = s_hist[d];
 }
 
-// Bucket starts and the segments of every bucket: ceil(size / seg_items)
-// segments, at least one (which writes the zeros of an empty bucket).  One
-// workgroup; n_seg = seg_first[nd] segments in all.
+// Bucket starts and the segments of every bucket (scatter_bucket_segments).
+// One workgroup; n_seg = seg_first[nd] segments in all.
 __global__ __launch_bounds__(256) void scatter_plan_kernel(const uint32_t* __restrict__ totals, int nd,
                                                            uint32_t seg_items, uint32_t* __restrict__ bucket_start,
                                                            uint32_t* __restrict__ seg_first,
@@ -210,7 +210,7 @@ __global__ __launch_bounds__(256) void scatter_plan_kernel(const uint32_t* __res
     if (d0 + j < nd) {
       const uint32_t c = totals[d0 + j];
       items += c;
-      segs += c == 0 ? 1 : (c + seg_items - 1) / seg_items;
+      segs += scatter_bucket_segments(c, seg_items);
     }
   int64_t all;
   int64_t run = block_exclusive_scan(items, s_wave, all);
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(256) void scatter_plan_kernel(const uint32_t* __res
   for (int j = 0; j < q; ++j)
     if (d0 + j < nd) {
       const uint32_t c = totals[d0 + j];
-      const int64_t k = c == 0 ? 1 : (c + seg_items - 1) / seg_items;
+      const int64_t k = scatter_bucket_segments(c, seg_items);
       bucket_start[d0 + j] = (uint32_t)run;
       seg_first[d0 + j] = (uint32_t)seg;
       for (int64_t u = 0; u < k; ++u) seg_bucket[seg + u] = (uint32_t)(d0 + j);
@@ -610,11 +610,7 @@ inline bool scatter_layout(int val_t, int64_t n_out, int64_t nnz, ScatterLayout&
   const int64_t nd = int64_t(1) << L.high_bits;
   L.waves = 4;
   while (L.waves > 1 && (acc << L.low_bits) * (size_t)L.waves > 65536) L.waves >>= 1;
-  // segments: enough to fill the chip, but a bucket of ordinary size whole
-  const int64_t used = ceil_div(n_out, int64_t(1) << L.low_bits);
-  const int64_t fill = std::max<int64_t>(2048, nnz / 1024);
-  const int64_t typical = nnz / used + nnz / used / 2;
-  L.seg_items = (uint32_t)(typical <= 4 * fill ? std::max(fill, typical) : fill);
+  L.seg_items = scatter_segment_items(nnz, ceil_div(n_out, int64_t(1) << L.low_bits));
   L.max_segs = nd + ceil_div(nnz, (int64_t)L.seg_items);
   L.n_tiles = ceil_div(nnz, kWgTile);
   L.n_sub = ceil_div(nnz, kWgSub);
