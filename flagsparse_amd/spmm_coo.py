@@ -134,8 +134,6 @@ def flagsparse_spmm_coo(data, row, col, B, shape, block_n=None, block_nnz=256, o
     data, row, col, B, n_rows, n_cols, n_dense = _prepare_spmm_coo_inputs(data, row, col, B, shape)
     if out is not None:
         _check_out(out, data.device, n_rows, n_dense, data.dtype)
-    if block_nnz is not None and block_nnz <= 0:
-        raise ValueError("block_nnz must be positive when provided")
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     # float16 / bfloat16 values are sorted as float32, which holds them exactly

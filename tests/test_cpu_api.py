@@ -266,18 +266,6 @@ def test_coo_validation_before_launch_on_cpu_tensors():
         fs.flagsparse_spmm_coo(d, i, i, B, (2, 2), op="trans")
 
 
-def test_coo_spmm_refuses_block_nnz_below_one(monkeypatch):
-    import flagsparse_amd.spmm_coo as spmm_coo_mod
-
-    one = torch.ones(1)
-    index = torch.zeros(1, dtype=torch.int32)
-    monkeypatch.setattr(spmm_coo_mod, "_prepare_spmm_coo_inputs",
-                        lambda *a: (one, index, index, one.view(1, 1), 1, 1, 1))
-    for bad in (0, -3):
-        with pytest.raises(ValueError, match="block_nnz must be positive when provided"):
-            fs.flagsparse_spmm_coo(one, index, index, one.view(1, 1), (1, 1), block_nnz=bad)
-
-
 def test_coo_int32_fallback_with_injected_launcher(monkeypatch):
     """spmv_coo.py:701-723 with an injected failing launch (CPU tensors, no
     device work): auto retries on int32 indices, strict re-raises, and an
