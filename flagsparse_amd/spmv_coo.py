@@ -22,6 +22,7 @@ complex128 (the reference accumulates both in single precision,
 spmv_coo.py:192-355; the results agree within its tolerances).
 """
 
+import os
 import time
 
 import torch
@@ -415,7 +416,9 @@ def flagsparse_spmv_coo(
     """COO SpMV y = op(A) @ x (spmv_coo.py:726-810).
 
     block_size / num_warps / block_inner keep the reference's validation;
-    the HIP kernels size their own tiles.  Returns y or (y, ms).
+    the HIP kernels size their own tiles.  Returns y or (y, ms): the time of
+    the launch on a prepared matrix, of the whole product with its index
+    checks for an unprepared call (which sorts nothing).
     """
     transpose_flag = False if transpose is None else bool(transpose)
     op_explicit = op is not None
@@ -504,7 +507,11 @@ def _spmv_coo_unsorted(data, row, col, x, shape, op_code, block_size, num_warps,
     the index ranges checked by the kernels and the reference's error
     (spmv_coo.py:390-422) raised before y is returned.  Returns (y, ms or
     None), or None when the general path must run: anything it would refuse,
-    empty shapes, float16 / bfloat16, or sizes the scatter does not take."""
+    empty shapes, sizes the scatter does not take, or a kernel forced by
+    FLAGSPARSE_SPMV_KERNEL or FLAGSPARSE_SPMV_ONESHOT=0 (as in
+    flagsparse_spmv_csr)."""
+    if os.environ.get("FLAGSPARSE_SPMV_ONESHOT", "1") == "0" or os.environ.get("FLAGSPARSE_SPMV_KERNEL"):
+        return None
     if not all(torch.is_tensor(t) for t in (data, row, col, x)):
         return None
     n_rows, n_cols = int(shape[0]), int(shape[1])

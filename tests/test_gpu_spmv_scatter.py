@@ -100,6 +100,21 @@ def test_largest_output_counts_take_or_leave_the_path():
     assert torch.allclose(y2[:n], y, rtol=1e-6, atol=1e-6)
 
 
+@pytest.mark.parametrize("name,value", [("FLAGSPARSE_SPMV_KERNEL", "vector"), ("FLAGSPARSE_SPMV_ONESHOT", "0")])
+def test_coo_call_follows_the_switches(monkeypatch, name, value):
+    data, row, col = _coo(5000, 300, 200, torch.float64, torch.int32, torch.int32, 4)
+    x = S.vector(200, torch.float64, DEV, 2)
+    monkeypatch.delenv("FLAGSPARSE_SPMV_KERNEL", raising=False)
+    y = fs.flagsparse_spmv_coo(data, row, col, x, (300, 200))
+    assert _lib.last_kernel() == "scatter_reduce_kernel"
+    monkeypatch.setenv(name, value)
+    y2 = fs.flagsparse_spmv_coo(data, row, col, x, (300, 200))
+    assert _lib.last_kernel() != "scatter_reduce_kernel"
+    if value == "vector":
+        assert _lib.last_kernel() == "spmv_vector_kernel"
+    assert torch.allclose(y, y2, rtol=1e-12, atol=1e-12)
+
+
 def test_structure_errors_keep_their_order():
     d, i, p, sh = S.random_csr(300, 200, 0.05, torch.float32, torch.int32, DEV, seed=3)
     x = S.vector(300, torch.float32, DEV, 4)
