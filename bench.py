@@ -310,11 +310,11 @@ def run_config(name, args):
                                             3: "uint8 code of the offset from the row"}[sell.col_code]
             if sell.table is not None:
                 extra["sell_distinct_offsets"] = sell.n_codes
-        pan = prep._panels
-        if pan is not None and hasattr(pan, "place"):
+        pan, gather = prep._panels, prep._gather
+        if gather is not None:
             # two-phase gather: the timed call is the whole sequence (gather, region walk, fixup)
-            kernel_call = lambda: (pan.spmv(x, y), 0)[1]  # noqa: E731
-            extra["n_slices"] = pan.n_panels
+            kernel_call = lambda: (gather.spmv(x, y), 0)[1]  # noqa: E731
+            extra["n_slices"] = gather.n_slices
         elif pan is not None:
             # column panels: the timed call is the whole panel sequence
             # (block table, panel merge, fixup, panel reduction)
@@ -537,7 +537,7 @@ def _gather_floor_spmv(name, cfg, args, lib, device, stream):
 
     calls = []
     pan = prep._panels
-    if pan is not None and not hasattr(pan, "place"):
+    if pan is not None:
         pn = [int(pan.panel_nnz[q]) for q in range(pan.n_panels + 1)]
         isz = pan.indices.element_size()
         calls = [launcher(_lib.index_code(pan.indices.dtype), pan.indices.data_ptr(), isz, pn[q], pn[q + 1])

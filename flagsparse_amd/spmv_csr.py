@@ -109,6 +109,7 @@ class PreparedCsrSpmv:
         "_part",
         "_carry",
         "_panels",
+        "_gather",
         "_sell",
         "_opt",
         "_one_shot",
@@ -159,6 +160,7 @@ class PreparedCsrSpmv:
         self._part = None
         self._carry = None
         self._panels = None
+        self._gather = None
         self._sell = None
         self._opt = None  # row-length buckets of the use_opt path (built on first use)
         self._one_shot = False  # built for a single call: no column-panel copy
@@ -201,12 +203,12 @@ class PreparedCsrSpmv:
             worth = _spmv_gather_worth(p, data.element_size(), self._one_shot)
             if worth is not None:
                 try:
-                    self._panels = GatheredCsr.build(data, self.kernel_indices, self.kernel_indptr, self.n_rows,
+                    self._gather = GatheredCsr.build(data, self.kernel_indices, self.kernel_indptr, self.n_rows,
                                                      self.n_cols, self._plan, worth)
                 except torch.OutOfMemoryError:
-                    self._panels = None
+                    self._gather = None
                     torch.cuda.empty_cache()
-                if self._panels is not None:
+                if self._gather is not None:
                     return self._plan
             if p.kernel == _lib.FS_KERNEL_MERGE:
                 n_panels = _spmv_panel_count(p, data.dtype, self._one_shot)
@@ -238,7 +240,7 @@ class PreparedCsrSpmv:
         if p.kernel == _lib.FS_KERNEL_MERGE:
             self._part = self._plan.partition(self.kernel_indptr, int(p.tile_items))
             self._carry = _lib.workspace(p.carry_bytes, self.data.device)
-        self._panels = None
+        self._gather = None
 
     def compute_data(self):
         """Values in the dtype the kernel runs in (f16/bf16 -> f32, cached)."""
@@ -254,14 +256,15 @@ class PreparedCsrSpmv:
         plan = self.hip_plan()
         if self._sell is not None:
             return "sell"
+        if self._gather is not None:
+            return "gather"
         return "panel" if self._panels is not None else plan.kernel_name
 
 
-# Column panels (matrices that the two-phase gather below does not take:
-# complex128, columns beyond its slices) pay off once x is larger than an XCD's
-# 4 MiB L2: the random
-# gather rate measured on MI355X drops from ~150-190 to ~70 gathers/ns when
-# x (16.8 MB) no longer fits.  A panel slice of up to ~4.5 MiB measured best
+# Column panels (merge-path matrices that the two-phase gather below does not
+# take: complex128, columns beyond its slices, few long rows) pay off once x is
+# larger than an XCD's 4 MiB L2: the random gather rate measured on MI355X drops
+# from ~150-190 to ~70 gathers/ns when x (16.8 MB) no longer fits.  A panel slice of up to ~4.5 MiB measured best
 # (4 panels on a 16.8 MB x: 0.61 ms against 0.67 ms with 8 and 1.01 ms with
 # none) since every panel adds n_rows row ends and partials.
 _PANEL_X_BYTES = 6 << 20
@@ -391,11 +394,11 @@ class GatheredCsr:
     16-bit place of its x within its region and, in column-slice order, its
     16-bit column number; the values and the row pointer stay the caller's.
 
-    indices: the column numbers, two to an int32 word; indptr: the first quad
-    of every region."""
+    columns: the column numbers, two to an int32 word; slice_q / region_q: the
+    first quad of every slice (of the stream) and region."""
 
-    __slots__ = ("data", "csr_indptr", "n_cols", "part", "pos", "indices", "place", "slice_q", "indptr", "n_quads",
-                 "max_region_quads", "ws_bytes", "n_panels", "stream")
+    __slots__ = ("data", "indptr", "n_cols", "part", "pos", "columns", "place", "slice_q", "region_q", "n_slices",
+                 "n_quads", "max_region_quads", "ws_bytes", "stream")
 
     @classmethod
     def build(cls, data, indices, indptr, n_rows, n_cols, plan, worth):
@@ -425,19 +428,19 @@ class GatheredCsr:
         if not worth(regions, touched):
             return None
         self = cls()
-        self.data, self.csr_indptr, self.n_cols, self.part = data, indptr, n_cols, part
-        self.n_panels, self.n_quads, self.max_region_quads = n_slices, n_quads, max_quads
+        self.data, self.indptr, self.n_cols, self.part = data, indptr, n_cols, part
+        self.n_slices, self.n_quads, self.max_region_quads = n_slices, n_quads, max_quads
         self.ws_bytes = lib.fs_spmv_gather_workspace_bytes(val_t, n_rows, nnz, n_quads)
-        self.indptr = torch.zeros(regions + 1, dtype=torch.int32, device=device)
-        torch.cumsum(counts[0], 0, out=self.indptr[1:])
+        self.region_q = torch.zeros(regions + 1, dtype=torch.int32, device=device)
+        torch.cumsum(counts[0], 0, out=self.region_q[1:])
         self.slice_q = torch.zeros(n_slices + 1, dtype=torch.int32, device=device)
         torch.cumsum(totals, 0, out=self.slice_q[1:])
         self.pos = torch.empty(nnz, dtype=torch.int16, device=device)
-        self.indices = torch.empty(2 * n_quads, dtype=torch.int32, device=device)
+        self.columns = torch.empty(2 * n_quads, dtype=torch.int32, device=device)
         self.place = torch.empty(n_quads, dtype=torch.int32, device=device)
         _lib.check(
-            lib.fs_spmv_gather_fill(*args, _lib.ptr(ws), _lib.ptr(self.indptr), _lib.ptr(self.pos),
-                                    _lib.ptr(self.indices), _lib.ptr(self.place), stream),
+            lib.fs_spmv_gather_fill(*args, _lib.ptr(ws), _lib.ptr(self.region_q), _lib.ptr(self.pos),
+                                    _lib.ptr(self.columns), _lib.ptr(self.place), stream),
             "fs_spmv_gather_fill",
         )
         # calls on other streams store at the places this wrote: without a
@@ -455,15 +458,15 @@ class GatheredCsr:
             # a dropped plan's memory waits for the calls still queued here: its
             # next owner would overwrite their store places
             current = torch.cuda.current_stream(device)
-            for t in (self.part, self.pos, self.indices, self.place, self.slice_q, self.indptr):
+            for t in (self.part, self.pos, self.columns, self.place, self.slice_q, self.region_q):
                 t.record_stream(current)
         ws = _lib.workspace(self.ws_bytes, device)
         _lib.check(
             _lib.lib().fs_spmv_csr_gather(
-                _lib.value_code(self.data.dtype), _lib.index_code(self.csr_indptr.dtype), self.csr_indptr.numel() - 1,
-                self.n_cols, self.data.numel(), _lib.ptr(self.data), _lib.ptr(self.csr_indptr), _lib.ptr(x),
-                _lib.ptr(y), _lib.ptr(self.part), _lib.ptr(self.pos), _lib.ptr(self.indices), _lib.ptr(self.place),
-                _lib.ptr(self.slice_q), _lib.ptr(self.indptr), self.n_quads, self.max_region_quads, _lib.ptr(ws),
+                _lib.value_code(self.data.dtype), _lib.index_code(self.indptr.dtype), self.indptr.numel() - 1,
+                self.n_cols, self.data.numel(), _lib.ptr(self.data), _lib.ptr(self.indptr), _lib.ptr(x),
+                _lib.ptr(y), _lib.ptr(self.part), _lib.ptr(self.pos), _lib.ptr(self.columns), _lib.ptr(self.place),
+                _lib.ptr(self.slice_q), _lib.ptr(self.region_q), self.n_quads, self.max_region_quads, _lib.ptr(ws),
                 ws.numel(), stream,
             ),
             "fs_spmv_csr_gather",
@@ -1089,7 +1092,7 @@ def _hip_spmv_csr_impl_prepared(prepared, x):
     x_in = x if x.dtype == cdt else x.to(cdt)
     y_out = y if cdt == dtype else torch.empty(prepared.n_rows, dtype=cdt, device=device)
     plan = prepared.hip_plan()
-    copy = prepared._sell if prepared._sell is not None else prepared._panels
+    copy = prepared._sell or prepared._gather or prepared._panels
     if copy is not None:
         try:
             copy.spmv(x_in, y_out)

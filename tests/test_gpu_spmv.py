@@ -310,19 +310,23 @@ def test_spmv_full_size_configs(device, config):
 
 @pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64], ids=["int32", "int64"])
 def test_spmv_panels_match_unpanelled(device, monkeypatch, index_dtype):
-    """Power-law matrix at the BASELINE size: the column-panel path (chosen by
-    default there) agrees with the single-pass merge path and the oracle on
-    sampled rows, and is deterministic.  int64 input is stacked with int32
-    indices (the stacked copy is internal; the caller's tensors keep int64)."""
+    """Power-law matrix at the BASELINE size: the column-panel path (forced;
+    by default this one takes the two-phase gather) agrees with the single-pass
+    merge path and the oracle on sampled rows, and is deterministic.  int64
+    input is stacked with int32 indices (the stacked copy is internal; the
+    caller's tensors keep int64)."""
+    from flagsparse_amd.spmv_csr import PanelledCsr
+
     monkeypatch.delenv("FLAGSPARSE_SPMV_KERNEL", raising=False)
-    monkeypatch.delenv("FLAGSPARSE_SPMV_PANELS", raising=False)
+    monkeypatch.setenv("FLAGSPARSE_SPMV_PANELS", "4")
     data, indices, indptr, sh = S.powerlaw(4194304, torch.float32, index_dtype, device, seed=3)
     prep = fs.prepare_spmv_csr(data, indices, indptr, sh)
-    assert prep.kernel_name == "panel"
+    assert prep.kernel_name == "panel" and isinstance(prep._panels, PanelledCsr)
     assert prep._panels.indices.dtype == torch.int32 and prep._panels.indptr.dtype == torch.int32
     assert prep.kernel_indices.dtype == index_dtype
     x = S.vector(sh[1], data.dtype, device, seed=23)
     y = fs.flagsparse_spmv_csr(x=x, prepared=prep)
+    assert _lib.last_kernel() == "spmv_panel_pipe_kernel"
     assert torch.equal(y, fs.flagsparse_spmv_csr(x=x, prepared=prep))
     monkeypatch.setenv("FLAGSPARSE_SPMV_PANELS", "0")
     prep0 = fs.prepare_spmv_csr(data, indices, indptr, sh)
@@ -341,6 +345,26 @@ def test_spmv_panels_match_unpanelled(device, monkeypatch, index_dtype):
     gen = np.random.default_rng(1)
     rows = sorted(set(gen.integers(0, sh[0], 3000).tolist()) | {0, sh[0] - 1})
     _sampled_rows_check(data, indices, indptr, sh, x, y, rows, REL_TOL[data.dtype])
+
+
+# what the two-phase gather does not take: complex128, more than 256 slices of
+# 32768 float32 columns, few long rows over an x of more than 16 MiB
+@pytest.mark.parametrize("dtype,n_cols,n_panels", [
+    (torch.complex128, 600_000, 4), (torch.float32, (1 << 23) + 5, 8), (torch.float64, 4_000_000, 8),
+], ids=["c128", "many_columns", "long_rows"])
+def test_spmv_panels_chosen_by_default(device, monkeypatch, dtype, n_cols, n_panels):
+    from flagsparse_amd.spmv_csr import PanelledCsr
+
+    monkeypatch.delenv("FLAGSPARSE_SPMV_KERNEL", raising=False)
+    monkeypatch.delenv("FLAGSPARSE_SPMV_PANELS", raising=False)
+    data, indices, indptr, sh = S.uniform_rows(100_000, n_cols, 80, dtype, torch.int64, device, seed=5)
+    prep = fs.prepare_spmv_csr(data, indices, indptr, sh)
+    assert isinstance(prep._panels, PanelledCsr) and prep._panels.n_panels == n_panels and prep._gather is None
+    x = S.vector(n_cols, dtype, device, seed=24)
+    y, meta = fs.flagsparse_spmv_csr(x=x, prepared=prep, return_meta=True)
+    assert meta["kernel"] == "panel" and _lib.last_kernel() == "spmv_panel_pipe_kernel"
+    rows = np.random.default_rng(1).integers(0, sh[0], 2000).tolist()
+    _sampled_rows_check(data, indices, indptr, sh, x, y, rows, REL_TOL[dtype])
 
 
 @pytest.mark.parametrize("n_panels", [1, 2, 4, 8, 13, 64])

@@ -100,8 +100,10 @@ def test_chosen_by_spread_of_columns(monkeypatch):
     d, i, p, sh = S.uniform_rows(n, n, 8, torch.float32, torch.int32, DEV, seed=1)
     x = S.vector(n, torch.float32, DEV, 2)
     for op in ("non", "trans"):
-        fs.flagsparse_spmv_csr(x=x, prepared=fs.prepare_spmv_csr(d, i, p, sh, op=op))
+        prep = fs.prepare_spmv_csr(d, i, p, sh, op=op)
+        _, meta = fs.flagsparse_spmv_csr(x=x, prepared=prep, return_meta=True)
         assert _lib.last_kernel() == "spmv_region_kernel"
+        assert meta["kernel"] == prep.kernel_name == "gather" and prep._panels is None
     fs.flagsparse_spmv_csr(d, i, p, x, sh)
     assert _lib.last_kernel() == "spmv_oneshot_kernel"
     band = ((torch.arange(n, device=DEV).repeat_interleave(8) + i.long() % 30011) % n).int()

@@ -76,7 +76,7 @@ def test_a_call_on_another_stream_keeps_the_plan_alive(recorded, monkeypatch):
         def __getattr__(self, name):
             return getattr(self.t, name)
 
-    names = ("part", "pos", "indices", "place", "slice_q", "indptr")
+    names = ("part", "pos", "columns", "place", "slice_q", "region_q")
     for name in names:
         setattr(plan, name, Tensor(getattr(plan, name)))
     plan.spmv(x, y)
