@@ -18,6 +18,7 @@ import ctypes
 import os
 import threading
 import time
+import warnings
 
 import numpy as np
 import torch
@@ -233,14 +234,6 @@ class PreparedCsrSpmv:
                 )
                 self._carry = _lib.workspace(p.carry_bytes, data.device)
         return self._plan
-
-    def drop_gather(self):
-        """Leaves the two-phase gather for the one-pass kernel of the plan."""
-        p = self._plan.plan
-        if p.kernel == _lib.FS_KERNEL_MERGE:
-            self._part = self._plan.partition(self.kernel_indptr, int(p.tile_items))
-            self._carry = _lib.workspace(p.carry_bytes, self.data.device)
-        self._gather = None
 
     def compute_data(self):
         """Values in the dtype the kernel runs in (f16/bf16 -> f32, cached)."""
@@ -1092,23 +1085,26 @@ def _hip_spmv_csr_impl_prepared(prepared, x):
     x_in = x if x.dtype == cdt else x.to(cdt)
     y_out = y if cdt == dtype else torch.empty(prepared.n_rows, dtype=cdt, device=device)
     plan = prepared.hip_plan()
+    part, carry = prepared._part, prepared._carry
     copy = prepared._sell or prepared._gather or prepared._panels
     if copy is not None:
         try:
             copy.spmv(x_in, y_out)
         except torch.OutOfMemoryError:
-            # a gathered call's workspace is its own: without room for it the
-            # CSR kernels run, from here on
-            if not isinstance(copy, GatheredCsr):
+            if copy is not prepared._gather:
                 raise
-            torch.cuda.empty_cache()
-            prepared.drop_gather()
+            # a gathered call's workspace is its own: a call without room for it
+            # runs the plan's one-pass kernel (over the same partition, with a
+            # carry of its own); the next one gathers again
+            warnings.warn(f"no room for the {copy.ws_bytes}-byte workspace of a two-phase SpMV: this call runs in "
+                          f"one pass ({plan.kernel_name})", RuntimeWarning, stacklevel=2)
+            if plan.plan.kernel == _lib.FS_KERNEL_MERGE:
+                part, carry = copy.part, _lib.workspace(plan.plan.carry_bytes, device)
             copy = None
     if copy is not None:
         if y_out is not y:
             y.copy_(y_out)
         return y
-    carry = prepared._carry
     _lib.check(
         _lib.lib().fs_spmv_csr(
             plan.plan,
@@ -1117,7 +1113,7 @@ def _hip_spmv_csr_impl_prepared(prepared, x):
             _lib.ptr(prepared.kernel_indptr),
             _lib.ptr(x_in),
             _lib.ptr(y_out),
-            _lib.ptr(prepared._part),
+            _lib.ptr(part),
             _lib.ptr(carry),
             0 if carry is None else carry.numel(),
             _lib.stream_handle(device),

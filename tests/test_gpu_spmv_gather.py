@@ -163,11 +163,16 @@ def test_call_without_room_for_its_workspace(any_size, monkeypatch, lengths):
     def no_memory(self, x, y):
         raise torch.OutOfMemoryError("injected")
 
-    monkeypatch.setattr(spmv_mod.GatheredCsr, "spmv", no_memory)
-    for _ in range(2):
-        y = fs.flagsparse_spmv_csr(x=x, prepared=prep)
-        assert _lib.last_kernel() != "spmv_region_kernel"
-        assert torch.allclose(y, want, rtol=1e-6, atol=1e-6)
+    with monkeypatch.context() as m:
+        m.setattr(spmv_mod.GatheredCsr, "spmv", no_memory)
+        for _ in range(2):
+            with pytest.warns(RuntimeWarning, match="no room"):
+                y = fs.flagsparse_spmv_csr(x=x, prepared=prep)
+            assert _lib.last_kernel() != "spmv_region_kernel"
+            assert torch.allclose(y, want, rtol=1e-6, atol=1e-6)
+    # one call's shortage is not the matrix's
+    assert torch.equal(fs.flagsparse_spmv_csr(x=x, prepared=prep), want)
+    assert _lib.last_kernel() == "spmv_region_kernel" and prep.kernel_name == "gather"
 
 
 def test_replayed_from_a_graph(any_size):
