@@ -778,10 +778,14 @@ __global__ __launch_bounds__(256) void spmv_oneshot_kernel(
       // us a call against 1005, 1 M power-law rows float32 277 against 204.)
       constexpr int kShort = 64, kMid = 4096;
       const auto last = ColGuard<I>::last(nc);
-      // entries first, first + stride, ... below len of the row at S + a, N loads in flight
-      auto row_part = [&](auto n_tag, int a, int len, int first, int stride) -> A {
-        constexpr int N = decltype(n_tag)::value;
-        A acc = T::zero();
+      // entries first, first + stride, ... below len of the row at S + a, N loads
+      // in flight, each with a sum of its own (a wave's row is as many short
+      // chains as the workgroup's was: the same error bound)
+      auto row_part = [&](int a, int len, int first, int stride) -> A {
+        constexpr int N = 4;
+        A acc[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) acc[k] = T::zero();
         for (int q0 = first; q0 - first < len; q0 += N * stride) {
           V v[N], xv[N];
 #pragma unroll
@@ -794,27 +798,27 @@ __global__ __launch_bounds__(256) void spmv_oneshot_kernel(
           }
 #pragma unroll
           for (int k = 0; k < N; ++k)
-            if (q0 + k * stride < len) acc = T::fma(v[k], xv[k], acc);
+            if (q0 + k * stride < len) acc[k] = T::fma(v[k], xv[k], acc[k]);
         }
-        return acc;
+        return add(add(acc[0], acc[1]), add(acc[2], acc[3]));
       };
       const int lane = t & 63, w = t >> 6;
       for (int r = t >> 4; r < rows; r += 16) {
         const int a = s_off[r], len = s_off[r + 1] - a;
         if (len > kShort) continue;
-        const A sum = group_sum<16>(row_part(std::integral_constant<int, 4>{}, a, len, t & 15, 16));
+        const A sum = group_sum<16>(row_part(a, len, t & 15, 16));
         if ((t & 15) == 0) y[rb0 + r] = T::out(sum);
       }
       for (int r = w; r < rows; r += 4) {
         const int a = s_off[r], len = s_off[r + 1] - a;
         if (len <= kShort || len > kMid) continue;
-        const A sum = wave_total(row_part(std::integral_constant<int, 4>{}, a, len, lane, 64));
+        const A sum = wave_total(row_part(a, len, lane, 64));
         if (lane == 0) y[rb0 + r] = T::out(sum);
       }
       for (int r = 0; r < rows; ++r) {
         const int a = s_off[r], len = s_off[r + 1] - a;
         if (len <= kMid) continue;  // the same for the whole workgroup
-        const A sum = wave_total(row_part(std::integral_constant<int, 4>{}, a, len, t, 256));
+        const A sum = wave_total(row_part(a, len, t, 256));
         if (lane == 0) s_red[w] = sum;
         __syncthreads();
         if (t == 0) y[rb0 + r] = T::out(add(add(s_red[0], s_red[1]), add(s_red[2], s_red[3])));

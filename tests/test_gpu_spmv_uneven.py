@@ -51,3 +51,19 @@ def test_half_values(dtype, op):
     assert torch.equal(y, want)
     with pytest.raises(TypeError, match="x dtype must match"):
         fs.flagsparse_spmv_csr(d, i, p, x.float(), sh, op=op)
+
+
+@pytest.mark.parametrize("length", [1024, 2048, 4096])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.complex128], ids=["f64", "c128"])
+def test_rows_of_a_wave_sum_in_256_chains(dtype, length):
+    """1 + (length - 1) 2^-54: a chain that starts with the 1 loses each of its
+    later terms, and the other chains' sums are whole multiples of 2^-52, so the
+    result says how long a chain is."""
+    lengths = [length] * 32 + [3] * 32
+    _, i, p, sh = _matrix(torch.float64, torch.int32, lengths, 9000)
+    d = torch.full((int(p[-1]),), 2.0**-54, dtype=dtype, device=DEV)
+    d[p[:-1].long()] = 1.0
+    y = fs.flagsparse_spmv_csr(d, i, p, torch.ones(9000, dtype=dtype, device=DEV), sh)
+    assert _lib.last_kernel() == "spmv_oneshot_kernel"
+    lost = (length - 1) * 2.0**-54 - (np_(y)[:32].real - 1.0)
+    assert np.all(np.abs(lost) <= (length // 256 - 1) * 2.0**-54)
