@@ -379,9 +379,10 @@ def _hip_spmm(data, indices, indptr, B, n_rows, plan, out_dtype, C=None):
     """C = A @ B for a dense B of any non-negative strides (row-major,
     column-major or strided views); returns C.
 
-    C is written in place when it is given with the compute dtype, else a
-    row-major C is allocated.  Strides go to the kernel as they are: no copy
-    of B or C is made for column-major layouts."""
+    A given C is written in place, through a copy of its layout where the
+    compute dtype is another; else a row-major C is allocated.  Strides go to
+    the kernel as they are: no copy of B or C is made for column-major
+    layouts."""
     device = data.device
     n_dense = int(B.shape[1])
     # 16-bit values go to the kernel as they are, except wide B that it would
@@ -402,12 +403,14 @@ def _hip_spmm(data, indices, indptr, B, n_rows, plan, out_dtype, C=None):
     B_c = B if B.dtype == cdt else B.to(cdt)
     if any(st < 0 for st in B_c.stride()):
         B_c = B_c.contiguous()
-    if C is None or C.dtype != cdt:
+    if C is None:
         C_k = torch.empty((n_rows, n_dense), dtype=cdt, device=device)
+    elif C.dtype != cdt:
+        C_k = torch.empty_strided(C.shape, C.stride(), dtype=cdt, device=device)
     else:
         C_k = C
     if n_rows == 0 or n_dense == 0:
-        return C_k if cdt == out_dtype else C_k.to(out_dtype)
+        return C if C is not None else C_k.to(out_dtype)
     if sell is not None and sell.spmm_fits(B_c, C_k):
         sell.spmm(B_c, C_k)
     elif data.numel() == 0:
@@ -441,9 +444,9 @@ def _hip_spmm(data, indices, indptr, B, n_rows, plan, out_dtype, C=None):
             ),
             "fs_spmm_csr",
         )
-    if cdt != out_dtype:
-        return C_k.to(out_dtype)
-    return C_k
+    if C is not None:
+        return C if C_k is C else C.copy_(C_k)
+    return C_k if cdt == out_dtype else C_k.to(out_dtype)
 
 
 def flagsparse_spmm_csr(

@@ -58,6 +58,20 @@ def test_ops_and_layouts(dtype, op):
     _check(C, d, i, p, sh, B, op)
 
 
+# up to 64 columns in 16 bits, above through float32 (a column-major B)
+@pytest.mark.parametrize("n", [1, 48, 64, 65, 128])
+@pytest.mark.parametrize("dtype", HALF, ids=["f16", "bf16"])
+def test_column_major_result_at_any_width(dtype, n):
+    d, i, p, sh = _matrix(300, 500, 0.03, dtype, torch.int32, 4)
+    B = S.dense(500, n, torch.float32, DEV, 3).to(dtype)
+    route = fs.prepare_spmm_csr_route(d, i, p, sh)
+    C, meta = fs.flagsparse_spmm_csr_run(route, B, dense_layout="col", return_meta=True)
+    assert C.dtype == dtype and C.stride() == (1, 300) and meta["c_stride"] == (1, 300)
+    if n > 1:
+        assert meta["output_layout"] == "col"
+    _check(C, d, i, p, sh, B)
+
+
 @pytest.mark.parametrize("dtype", HALF, ids=["f16", "bf16"])
 def test_stencil_keeps_its_copy(dtype):
     """A prepared stencil runs on its float32 SELL-64 copy; widths it does not
