@@ -297,28 +297,78 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(
   }
 }
 
-// Rows that cross sub-tiles: C[row] = tail[f] + ... + tail[t-1] + head[t].
+// Rows that cross sub-tiles: C[row] = tail[f] + ... + tail[t-1] + head[t], one
+// wave per sub-tile t, lanes over columns.  A row of more than kFixShort
+// fragments is the workgroup's: its threads take columns x equal shares of the
+// fragments, joined in a fixed tree (of 16 sub-tiles in a row at most one ends
+// such a row: the next one to end started after it).  One wave adding them all
+// is a chain of loads that outlasts what small sub-tiles win.  us per prepared
+// float32 call on an arrow matrix of 100,000 rows (its dense row up to 3,125
+// fragments), 2048-item waves / sized sub-tiles, one wave / 4 waves / 16 waves:
+// N = 1 121 / 103 / 24 / 24, N = 17 145 / 142 / 52 / 46, N = 64 178 / 94 / 50 /
+// 43, N = 256 75 / 94 / 71 / 68; without long rows 16 waves cost nothing (1 M
+// rows of 30, N = 64 1130 / 1130; 4 waves 1135).
+constexpr int kFixWaves = 16;
+constexpr int kFixThreads = 64 * kFixWaves;
+constexpr int64_t kFixShort = 32;
 template <class V, class T = VT<V>>
-__global__ __launch_bounds__(256) void spmm_group_fixup_kernel(
+__global__ __launch_bounds__(kFixThreads) void spmm_group_fixup_kernel(
     const void* __restrict__ rowptr_raw, int ptr64, const int64_t* __restrict__ part, int sub_items,
     const typename T::acc* __restrict__ head, const typename T::acc* __restrict__ tail,
     V* __restrict__ C, int64_t scm, int64_t scn, int64_t n_dense, int64_t n_sub) {
   using A = typename T::acc;
-  const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= n_sub) return;
-  const int64_t r0 = part[t];
-  if (part[t + 1] == r0) return;
-  const int64_t n0 = t * (int64_t)sub_items - r0;
-  const int64_t start = ptr64 ? static_cast<const int64_t*>(rowptr_raw)[r0]
-                              : (int64_t) static_cast<const int32_t*>(rowptr_raw)[r0];
-  if (start >= n0) return;
-  const int64_t f = fixup_start_tile(part, t, r0);
-  for (int64_t col = (int64_t)blockIdx.y * 64 + (threadIdx.x & 63); col < n_dense;
-       col += (int64_t)gridDim.y * 64) {
-    A sum = tail[f * n_dense + col];
-    sum = sum_fragments(tail + col, n_dense, f + 1, t, sum);  // in sub-tile order
-    sum = add(sum, head[t * n_dense + col]);
-    C[r0 * scm + col * scn] = T::out(sum);
+  __shared__ int64_t s_long[kFixWaves];  // per wave: the first sub-tile of a long row, or -1
+  __shared__ A s_sum[kFixThreads];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t t = (int64_t)blockIdx.x * kFixWaves + (tid >> 6);
+  int64_t long_f = -1;
+  if (t < n_sub) {
+    const int64_t r0 = part[t];
+    const bool ends = part[t + 1] != r0;
+    const int64_t n0 = t * (int64_t)sub_items - r0;
+    const int64_t start = !ends ? n0
+                          : ptr64 ? static_cast<const int64_t*>(rowptr_raw)[r0]
+                                  : (int64_t) static_cast<const int32_t*>(rowptr_raw)[r0];
+    if (start < n0) {
+      const int64_t f = fixup_start_tile(part, t, r0);
+      if (t - f > kFixShort) {
+        long_f = f;
+      } else {
+        for (int64_t col = (int64_t)blockIdx.y * 64 + lane; col < n_dense; col += (int64_t)gridDim.y * 64) {
+          A sum = tail[f * n_dense + col];
+          sum = sum_fragments(tail + col, n_dense, f + 1, t, sum);  // in sub-tile order
+          sum = add(sum, head[t * n_dense + col]);
+          C[r0 * scm + col * scn] = T::out(sum);
+        }
+      }
+    }
+  }
+  if (lane == 0) s_long[tid >> 6] = long_f;
+  __syncthreads();
+  const uint64_t found = __ballot(lane < kFixWaves && s_long[lane < kFixWaves ? lane : 0] >= 0);
+  if (found == 0) return;  // whole workgroup
+  const int lw = (int)__builtin_ctzll(found);
+  const int64_t lt = (int64_t)blockIdx.x * kFixWaves + lw, lf = s_long[lw], row = part[lt];
+  for (int64_t c0 = (int64_t)blockIdx.y * 64; c0 < n_dense; c0 += (int64_t)gridDim.y * 64) {
+    const int nc = n_dense - c0 < 64 ? (int)(n_dense - c0) : 64;
+    int width = 1;  // threads per share: the columns, rounded up to a power of two
+    while (width < nc) width <<= 1;
+    const int shares = kFixThreads / width, share = tid / width, c = tid % width;
+    const int64_t len = (lt - lf + shares - 1) / shares;
+    const int64_t k0 = lf + share * len < lt ? lf + share * len : lt;
+    const int64_t k1 = lt - k0 < len ? lt : k0 + len;
+    A sum = T::zero();
+    if (c < nc) sum = sum_fragments(tail + c0 + c, n_dense, k0, k1, sum);
+    s_sum[tid] = sum;
+    for (int o = shares >> 1; o > 0; o >>= 1) {
+      __syncthreads();
+      if (share < o) s_sum[tid] = add(s_sum[tid], s_sum[tid + o * width]);
+    }
+    if (share == 0 && c < nc) {
+      sum = add(s_sum[tid], head[lt * n_dense + c0 + c]);
+      C[row * scm + (c0 + c) * scn] = T::out(sum);
+    }
+    __syncthreads();
   }
 }
 
@@ -365,10 +415,10 @@ int launch_spmm_group(const fs_csr_plan* plan, const void* vals, const void* col
   if (plan->idx_t == FS_I64) go(std::true_type{});
   else go(std::false_type{});
   FS_CHECK_MAIN_LAUNCH("spmm_group_kernel");
-  const int64_t fix_blocks = ceil_div(n_sub, 4);
+  const int64_t fix_blocks = ceil_div(n_sub, (int64_t)kFixWaves);
   const int64_t fix_cols = ceil_div(n_dense, 64) < 64 ? ceil_div(n_dense, 64) : 64;
-  hipLaunchKernelGGL((spmm_group_fixup_kernel<V, T>), dim3((unsigned)fix_blocks, (unsigned)fix_cols), dim3(256), 0,
-                     stream, indptr, plan->ptr_t == FS_I64 ? 1 : 0, part, sub_items, head, tail,
+  hipLaunchKernelGGL((spmm_group_fixup_kernel<V, T>), dim3((unsigned)fix_blocks, (unsigned)fix_cols),
+                     dim3(kFixThreads), 0, stream, indptr, plan->ptr_t == FS_I64 ? 1 : 0, part, sub_items, head, tail,
                      static_cast<V*>(C), scm, scn, n_dense, n_sub);
   FS_CHECK_LAUNCH("spmm_group_fixup_kernel");
   return FS_OK;

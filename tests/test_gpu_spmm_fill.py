@@ -31,6 +31,33 @@ def test_small_matrices(dtype, rows, long_rows, n):
     assert torch.equal(torch.view_as_real(C) if C.is_complex() else C, torch.view_as_real(Ct) if C.is_complex() else Ct)
 
 
+# 32 items a sub-tile with 16 lanes a row: rows of 1024 entries cross about 32
+# of them, where the fix-up goes from one wave to a workgroup of 1024 threads
+@pytest.mark.parametrize("lengths", [[5, 1000, 2], [1010] * 3, [1023, 1, 1024, 1025, 0, 1090], [0, 40000, 3, 0, 0, 33000, 7],
+                                     [100000] + [2] * 500], ids=lambda v: f"{len(v)}rows{sum(v)}nnz")
+@pytest.mark.parametrize("n", [1, 3, 17, 64, 65, 200])
+@pytest.mark.parametrize("dtype", VALUE_DTYPES + [torch.bfloat16], ids=VALUE_IDS + ["bf16"])
+def test_long_rows_of_many_fragments(dtype, n, lengths):
+    """Whole values, so that every order of the sums gives the same bits."""
+    g = np.random.default_rng(len(lengths))
+    ptr = np.concatenate([[0], np.cumsum(lengths)])
+    cols = g.integers(0, 5000, ptr[-1])
+    top = 1 if dtype == torch.bfloat16 else 4
+    vals, B = g.integers(-top, top + 1, ptr[-1]), g.integers(-top, top + 1, (5000, n))
+    ref = np.zeros((len(lengths), n))
+    for r in range(len(lengths)):
+        s = slice(ptr[r], ptr[r + 1])
+        ref[r] = vals[s] @ B[cols[s]]
+    args = [torch.tensor(vals, device=DEV).to(dtype), torch.tensor(cols, device=DEV).int(),
+            torch.tensor(ptr, device=DEV).int()]
+    Bt = torch.tensor(B, device=DEV).to(dtype)
+    C = fs.flagsparse_spmm_csr(*args, Bt, (len(lengths), 5000))
+    want = torch.tensor(ref, device=DEV).to(dtype)
+    assert torch.equal(C, want)
+    route = fs.prepare_spmm_csr_route(*args, (len(lengths), 5000))
+    assert torch.equal(fs.flagsparse_spmm_csr_run(route, Bt), want)
+
+
 def test_sizes_shrink_with_the_matrix_only():
     lib = _lib.lib()
     for n in (1, 32, 64, 128, 256):
