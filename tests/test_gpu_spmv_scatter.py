@@ -88,6 +88,23 @@ def test_hub_columns_and_split_buckets(dtype):
     assert rel_err(np_(y), ref) <= REL_TOL[dtype]
 
 
+@pytest.mark.parametrize("run", [1, 2, 5, 6, 7, 8, 13, 20, 31, 32, 63, 64, 65, 200])
+@pytest.mark.parametrize("nnz", [50, 64, 4001, 50000])
+@pytest.mark.parametrize("dtype", VALUE_DTYPES, ids=VALUE_IDS)
+def test_groups_of_equal_outputs(dtype, nnz, run):
+    """Runs of one output: groups of every size among a wave's lanes, alone and
+    several at once.  Whole values, so that every order gives the same bits."""
+    g = np.random.default_rng(run)
+    out = np.repeat(g.integers(0, 300, -(-nnz // run)), run)[:nnz]
+    src = g.integers(0, 40, nnz)
+    val, x = g.integers(-9, 10, nnz), g.integers(-9, 10, 40)
+    ref = np.bincount(out, weights=(val * x[src]).astype(np.float64), minlength=300)
+    args = [torch.tensor(v, device=DEV) for v in (val, out, src, x)]
+    y = fs.flagsparse_spmv_coo(args[0].to(dtype), args[1].int(), args[2], args[3].to(dtype), (300, 40))
+    assert _lib.last_kernel() == "scatter_reduce_kernel"
+    assert np.array_equal(np_(y), ref.astype(np_(y).dtype))
+
+
 def test_largest_output_counts_take_or_leave_the_path():
     n = 1 << 23
     data, row, col = _coo(50000, n, 9, torch.float32, torch.int32, torch.int32, 1)
