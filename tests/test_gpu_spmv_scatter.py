@@ -105,6 +105,22 @@ def test_groups_of_equal_outputs(dtype, nnz, run):
     assert np.array_equal(np_(y), ref.astype(np_(y).dtype))
 
 
+@pytest.mark.parametrize("n_out", [1, 3, 64, 100, 300, 1025])
+@pytest.mark.parametrize("dtype", VALUE_DTYPES, ids=VALUE_IDS)
+def test_buckets_of_many_segments(dtype, n_out):
+    """Up to 1,024 segments in a bucket, most entries in the last one.  Whole
+    values, so that every order gives the same bits."""
+    g = np.random.default_rng(n_out)
+    nnz = 2_200_001
+    out = n_out - 1 - (g.random(nnz) ** 4 * n_out).astype(np.int64)
+    src, val, x = g.integers(0, 40, nnz), g.integers(-2, 3, nnz), g.integers(-2, 3, 40)
+    ref = np.bincount(out, weights=(val * x[src]).astype(np.float64), minlength=n_out)
+    args = [torch.tensor(v, device=DEV) for v in (val, out, src, x)]
+    y = fs.flagsparse_spmv_coo(args[0].to(dtype), args[1].int(), args[2].int(), args[3].to(dtype), (n_out, 40))
+    assert _lib.last_kernel() == "scatter_reduce_kernel"
+    assert np.array_equal(np_(y), ref.astype(np_(y).dtype))
+
+
 def test_largest_output_counts_take_or_leave_the_path():
     n = 1 << 23
     data, row, col = _coo(50000, n, 9, torch.float32, torch.int32, torch.int32, 1)
