@@ -1450,10 +1450,15 @@ def _spmv_transposed_oneshot(data, indices, indptr, x, shape, op_code, index_fal
     return y
 
 
-# float16 / bfloat16 take the one-launch call while a call is what counts (3000
-# rows of 10: 83 us on the general path, 36 in one launch); above, hub rows
-# would cost more than its saved launches (R-MAT 2^20: 226 against 816 us).
+# float16 / bfloat16 take the one-launch call while a call is what counts (us,
+# general path / one launch: 3000 rows of 10 83 / 36, 16,384 of 15 91 / 37);
+# above, hub rows would cost more than its saved launches (R-MAT 2^20: 226 /
+# 816), and so do few long rows, which one workgroup walks (20 rows of 12,000
+# 103 / 222, one of 200,000 102 / 210; one of 60,000 98 / 84, 5 of 13,000 98 /
+# 89): up to 2^16 entries, or 2^18 where rows average at most 64.
+_ONESHOT_HALF_ANY_NNZ = 1 << 16
 _ONESHOT_HALF_MAX_NNZ = 1 << 18
+_ONESHOT_HALF_ROW = 64
 
 
 def _spmv_oneshot(data, indices, indptr, x, shape, index_fallback_policy, timed):
@@ -1462,8 +1467,8 @@ def _spmv_oneshot(data, indices, indptr, x, shape, index_fallback_policy, timed)
     errors are raised here, in its order (spmv_csr.py:546-558), before y
     is returned or `out` is written.  Returns (y, compute_ms) or None when
     the general path must run: an invalid x (its error comes after the
-    structure checks), empty shapes, large float16 / bfloat16, a forced
-    kernel, or a failed launch (the general path holds the int64 -> int32 fallback)."""
+    structure checks), empty shapes, float16 / bfloat16 of many entries or
+    long rows, a forced kernel, or a failed launch (the general path holds the int64 -> int32 fallback)."""
     if os.environ.get("FLAGSPARSE_SPMV_ONESHOT", "1") == "0" or os.environ.get("FLAGSPARSE_SPMV_KERNEL"):
         return None
     data, indices, indptr, n_rows, n_cols = _validate_spmv_host(data, indices, indptr, shape, index_fallback_policy)
@@ -1475,7 +1480,7 @@ def _spmv_oneshot(data, indices, indptr, x, shape, index_fallback_policy, timed)
     except (TypeError, ValueError):
         return None
     if data.dtype not in HIP_VALUE_DTYPES:  # float16 / bfloat16: computed in float32 (_compute_dtype)
-        if nnz > _ONESHOT_HALF_MAX_NNZ:
+        if nnz > max(_ONESHOT_HALF_ANY_NNZ, min(_ONESHOT_HALF_MAX_NNZ, _ONESHOT_HALF_ROW * n_rows)):
             return None
         cdt = _compute_dtype(data.dtype)
         done = _spmv_oneshot(data.to(cdt), indices, indptr, x.to(cdt), shape, index_fallback_policy, timed)

@@ -67,3 +67,18 @@ def test_rows_of_a_wave_sum_in_256_chains(dtype, length):
     assert _lib.last_kernel() == "spmv_oneshot_kernel"
     lost = (length - 1) * 2.0**-54 - (np_(y)[:32].real - 1.0)
     assert np.all(np.abs(lost) <= (length // 256 - 1) * 2.0**-54)
+
+
+@pytest.mark.parametrize("rows,per_row,one_launch", [
+    (16384, 16, True), (16384, 17, False), (4096, 64, True), (4096, 65, False), (4000, 65, False), (1, 65536, True),
+    (1, 65537, False), (20, 12000, False), (1024, 64, True), (100, 655, True),
+])
+def test_half_values_of_long_rows_take_the_general_path(rows, per_row, one_launch):
+    d, i, p, sh = _matrix(torch.float32, torch.int32, [per_row] * rows, 70001)
+    d = d.bfloat16()
+    x = S.vector(sh[1], torch.float32, DEV, 5).bfloat16()
+    y, meta = fs.flagsparse_spmv_csr(d, i, p, x, sh, return_meta=True)
+    assert (meta["kernel"] == "oneshot") == one_launch
+    want = torch.from_numpy(O.spmv_csr_wide(np_(d.double()), np_(i), np_(p), np_(x.double()), sh)).float().bfloat16()
+    # the same sums in another order may round to the next value
+    assert bool(((y.cpu().double() - want.double()).abs() <= want.double().abs() * 2.0**-7).all())
