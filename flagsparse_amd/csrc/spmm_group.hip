@@ -113,16 +113,29 @@ inline int spmm_tile_items_for(int val_t, int64_t n_dense) {
 // 75 / 45 / 37 / 39 / 50, N = 64 118 / 69 / 85 / 75 / 75; 300,000 of 20, f32,
 // N = 32: 128 / 128 / 128 / 137 / 149, f64, N = 32: 295 / 295 / 295 / 280 /
 // 253.  Smaller sub-tiles cost row fragments, more for narrow B rows: at least
-// 2048 waves there, 4096 with 32 lanes or more per row.
+// 2048 waves there, 4096 with 32 lanes or more per row.  With 32 lanes, whole
+// slices and short rows, 2048 to 3072 waves stay as they are: they run at once
+// (3 a SIMD), and half the size would be a round and a third of them.  us, as
+// they are / halved: 600,000 rows of 6, 2049 waves, f32 N = 64 166 / 191, f64 N =
+// 32 160 / 188; 400,009 of 10 174 / 186, 175 / 183; 100,000 of 10 (512 items)
+// 49 / 53, 48 / 52; but 600,000 of 10 (3221 waves) 350 / 293, 44,000 of 50 c128
+// N = 16 99 / 86, and at N = 33 (element loads) 400,009 of 10 289 / 242.
 constexpr int kGroupMinWaveItems = 128;
+constexpr int64_t kGroupSlots = 3072;
 inline int spmm_tile_items_sized(int val_t, int64_t n_dense, int64_t n_rows, int64_t nnz) {
   const int base = spmm_tile_items_for(val_t, n_dense);
   if (forced_kernel() != 0 || std::getenv("FLAGSPARSE_SPMM_WAVE_ITEMS")) return base;
   if (wide_rows(val_t, n_dense) && nnz >= kGroupSkewNnz) return base;
   const int lpr = group_lpr(val_t, n_dense);
   const int64_t fill = lpr >= 32 ? 4096 : 2048;
+  const int bytes = spmm_value_bytes(val_t);
+  const bool one_round = lpr == 32 && !spmm_half(val_t) && n_dense % (16 / bytes) == 0 &&
+                         nnz / (bytes == 16 ? 12 : 24) <= n_rows;
   int wave_items = base * 64 / lpr;
-  while (wave_items > kGroupMinWaveItems && ceil_div(n_rows + nnz, (int64_t)wave_items) < fill) wave_items >>= 1;
+  for (; wave_items > kGroupMinWaveItems; wave_items >>= 1) {
+    const int64_t waves = ceil_div(n_rows + nnz, (int64_t)wave_items);
+    if (waves >= fill || (one_round && waves >= 2048 && waves <= kGroupSlots)) break;
+  }
   return wave_items * lpr / 64;
 }
 

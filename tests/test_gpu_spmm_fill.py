@@ -69,6 +69,19 @@ def test_sizes_shrink_with_the_matrix_only():
     assert lib.fs_spmm_tile_items_sized(_lib.FS_F32, 128, 10, 1 << 20) == 512
 
 
+def test_one_round_of_waves_is_not_halved():
+    """Short rows, whole slices, 32 lanes a row (N = 64 in float32): 2048 to
+    3072 waves stay (32 lanes: half of a wave's items are a sub-tile's)."""
+    size = lambda t, n, rows, nnz: _lib.lib().fs_spmm_tile_items_sized(t, n, rows, nnz)  # noqa: E731
+    assert size(_lib.FS_F32, 64, 400_000, 4_000_000) == 1024  # 2149 waves of 2048
+    assert size(_lib.FS_F32, 64, 600_000, 6_000_000) == 512  # 3223: two rounds, halved
+    assert size(_lib.FS_F32, 64, 100_000, 1_000_000) == 256  # 2149 waves of 512
+    assert size(_lib.FS_F32, 33, 400_000, 4_000_000) == 512  # element loads
+    assert size(_lib.FS_F32, 64, 90_000, 4_300_000) == 512  # rows of 48
+    assert size(_lib.FS_C128, 16, 400_000, 4_000_000) == 1024
+    assert size(_lib.FS_C128, 16, 200_000, 4_000_000) == 512  # rows of 20
+
+
 def test_either_tile_size_is_taken():
     """A caller that sizes its partition by fs_spmm_tile_items is served as before."""
     d, i, p, sh = S.random_csr(500, 400, 0.03, torch.float32, torch.int32, DEV, seed=2)
