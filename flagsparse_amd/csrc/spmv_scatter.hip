@@ -42,6 +42,7 @@
 // with the structure is reported through the flags and the caller discards y.
 #include "fs_common.hpp"
 #include "radix_tile.hpp"
+#include "row_starts.hpp"
 #include "scatter_segments.hpp"
 
 #include <algorithm>
@@ -147,9 +148,8 @@ __global__ __launch_bounds__(256) void scatter_rows_kernel(const P* __restrict__
   if (r == 0 && a != 0) raise_flag(flags, 0);
   if (r == n_rows - 1 && b != nnz) raise_flag(flags, 1);
   if (b < a) raise_flag(flags, 2);
-  int64_t sub = a <= 0 ? 0 : (a + kWgSub - 1) / kWgSub;
-  const int64_t end = b <= 0 ? 0 : ((b + kWgSub - 1) / kWgSub < n_sub ? (b + kWgSub - 1) / kWgSub : n_sub);
-  for (; sub < end; ++sub) tile_row[sub] = r;
+  const int64_t end = row_sub_tile(b, kWgSub, n_sub);
+  for (int64_t sub = row_sub_tile(a, kWgSub, n_sub); sub < end; ++sub) tile_row[sub] = r;
 }
 
 // Bucket counts of every tile, cnt[tile][bucket], and the range check of the

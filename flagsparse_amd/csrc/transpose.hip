@@ -24,6 +24,7 @@
 //    the sorted keys (radix_* kernels).
 #include "fs_common.hpp"
 #include "radix_tile.hpp"
+#include "row_starts.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -711,9 +712,8 @@ __global__ __launch_bounds__(256) void wg_tile_rows_kernel(const P* __restrict__
   if (r >= n_rows) return;
   const int64_t a = (int64_t)rowptr[r], b = (int64_t)rowptr[r + 1];
   if (check != nullptr && b < a) atomicAdd(&check[2], 1ull);  // malformed input only
-  int64_t sub = a <= 0 ? 0 : (a + kWgSub - 1) / kWgSub;
-  const int64_t end = b <= 0 ? 0 : ((b + kWgSub - 1) / kWgSub < n_sub ? (b + kWgSub - 1) / kWgSub : n_sub);
-  for (; sub < end; ++sub) tile_row[sub] = r;
+  const int64_t end = row_sub_tile(b, kWgSub, n_sub);
+  for (int64_t sub = row_sub_tile(a, kWgSub, n_sub); sub < end; ++sub) tile_row[sub] = r;
 }
 
 // The fused structure check's column test over one lane's column values

@@ -194,3 +194,14 @@ def test_infinities_and_unaligned_views(dtype):
     fin = np.isfinite(ref)
     assert np.array_equal(np_(y)[~fin].astype(np.float64), ref[~fin], equal_nan=True)
     np.testing.assert_allclose(np_(y)[fin], ref[fin], rtol=1e-6, atol=1e-5)
+
+
+@pytest.mark.parametrize("n_cols", [200, (1 << 23) + 1], ids=["scatter", "transpose"])
+@pytest.mark.parametrize("value", [2**63 - 1, 2**63 - 700, 2**40, -(2**63)])
+def test_row_pointers_of_any_value_are_refused(value, n_cols):
+    """64-bit row pointers near the largest value: the structure error, from both ways to A^T x."""
+    d, i, p, _ = S.random_csr(300, 200, 0.05, torch.float32, torch.int64, DEV, seed=3)
+    p = p.long().clone()
+    p[100] = value
+    with pytest.raises(ValueError, match="non-decreasing"):
+        fs.flagsparse_spmv_csr(d, i, p, S.vector(300, torch.float32, DEV, 4), (300, n_cols), op="trans")
