@@ -300,17 +300,20 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(
 // Rows that cross sub-tiles: C[row] = tail[f] + ... + tail[t-1] + head[t], one
 // wave per sub-tile t, lanes over columns.  A row of more than kFixShort
 // fragments is the workgroup's: its threads take columns x equal shares of the
-// fragments, joined in a fixed tree (of 16 sub-tiles in a row at most one ends
-// such a row: the next one to end started after it).  One wave adding them all
-// is a chain of loads that outlasts what small sub-tiles win.  us per prepared
-// float32 call on an arrow matrix of 100,000 rows (its dense row up to 3,125
-// fragments), 2048-item waves / sized sub-tiles, one wave / 4 waves / 16 waves:
-// N = 1 121 / 103 / 24 / 24, N = 17 145 / 142 / 52 / 46, N = 64 178 / 94 / 50 /
-// 43, N = 256 75 / 94 / 71 / 68; without long rows 16 waves cost nothing (1 M
-// rows of 30, N = 64 1130 / 1130; 4 waves 1135).
-constexpr int kFixWaves = 16;
+// fragments, joined in a fixed tree (of kFixWaves sub-tiles in a row at most one
+// ends such a row: the next one to end started after it).  One wave adding them
+// all is a chain of loads that outlasts what small sub-tiles win.  us per
+// prepared float32 call on an arrow matrix of 100,000 rows (its dense row up to
+// 3,125 fragments), 2048-item waves / sized sub-tiles, one wave / 4 waves / 16
+// waves: N = 1 121 / 103 / 25 / 24, N = 17 145 / 142 / 52 / 46, N = 64 178 / 94 /
+// 50 / 43, N = 256 75 / 94 / 71 / 68.  4 waves, and only rows of more than 128
+// fragments: a workgroup of 16 is kept by its slowest wave, and with rows of
+// more than 32 on it the fix-up of an R-MAT graph went from 12 to 18 us (2^19,
+// N = 3, one wave / 4 / 16: 451 / 453 / 455 us a call; 2^21 complex64, N = 32 1393
+// / 1394 / 1396).
+constexpr int kFixWaves = 4;
 constexpr int kFixThreads = 64 * kFixWaves;
-constexpr int64_t kFixShort = 32;
+constexpr int64_t kFixShort = 128;
 template <class V, class T = VT<V>>
 __global__ __launch_bounds__(kFixThreads) void spmm_group_fixup_kernel(
     const void* __restrict__ rowptr_raw, int ptr64, const int64_t* __restrict__ part, int sub_items,

@@ -31,9 +31,10 @@ def test_small_matrices(dtype, rows, long_rows, n):
     assert torch.equal(torch.view_as_real(C) if C.is_complex() else C, torch.view_as_real(Ct) if C.is_complex() else Ct)
 
 
-# 32 items a sub-tile with 16 lanes a row: rows of 1024 entries cross about 32
-# of them, where the fix-up goes from one wave to a workgroup of 1024 threads
-@pytest.mark.parametrize("lengths", [[5, 1000, 2], [1010] * 3, [1023, 1, 1024, 1025, 0, 1090], [0, 40000, 3, 0, 0, 33000, 7],
+# 32 items a sub-tile with 16 lanes a row: rows of 4096 entries cross about 128
+# of them, where the fix-up goes from one wave to a workgroup
+@pytest.mark.parametrize("lengths", [[5, 1000, 2], [1010] * 3, [1023, 1, 1024, 1025, 0, 1090],
+                                     [4095, 1, 4096, 4097, 0, 4160], [0, 40000, 3, 0, 0, 33000, 7],
                                      [100000] + [2] * 500], ids=lambda v: f"{len(v)}rows{sum(v)}nnz")
 @pytest.mark.parametrize("n", [1, 3, 17, 64, 65, 200])
 @pytest.mark.parametrize("dtype", VALUE_DTYPES + [torch.bfloat16], ids=VALUE_IDS + ["bf16"])
