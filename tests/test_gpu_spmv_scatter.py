@@ -3,6 +3,8 @@
 segment edges, output counts from one bucket to thousands, crowded outputs,
 structure errors, special values and determinism."""
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -30,6 +32,50 @@ def _wide(data, row, col, x, n_out):
     p = np_(data).astype(np.complex128) * np_(x).astype(np.complex128)[np_(col)]
     re = np.bincount(np_(row), weights=p.real, minlength=n_out)
     return re + 1j * np.bincount(np_(row), weights=p.imag, minlength=n_out)
+
+
+def _cancelling(nnz, n_out, n_x, cplx, seed):
+    """Entries whose products are exact in float64 (25-bit whole values times
+    powers of two; a complex x is real or imaginary) and of mixed sign, with the
+    exactly rounded sums, the sums of magnitudes and the entries per output."""
+    g = np.random.default_rng(seed)
+
+    def values(n):
+        return g.integers(-(2**25), 2**25, n) * 2.0 ** g.integers(-8, 9, n)
+
+    out, src = g.integers(0, n_out, nnz), g.integers(0, n_x, nnz)
+    val, x = values(nnz), values(n_x)
+    if cplx:
+        val = val + 1j * values(nnz)
+        x = np.where(np.arange(n_x) % 2 == 0, x + 0j, 1j * x)
+    terms = val * x[src]
+    order = np.argsort(out, kind="stable")
+    count = np.bincount(out, minlength=n_out)
+    parts = []
+    for t in (terms.real, terms.imag) if cplx else (terms,):
+        groups = np.split(t[order], np.cumsum(count)[:-1])
+        parts.append((np.array([math.fsum(p) for p in groups]), np.bincount(out, weights=np.abs(t), minlength=n_out),
+                      np.bincount(out, weights=t, minlength=n_out)))
+    return val, out, src, x, count, parts
+
+
+@pytest.mark.parametrize("n_out", [1, 3, 64, 2500, 300007])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.complex128], ids=["f64", "c128"])
+def test_double_sums_are_compensated(dtype, n_out):
+    """Two roundings (2 u |sum|, u = 2^-53) and the rounding of the compensation
+    itself (at most n terms of u times the sum of magnitudes, added with another
+    n u): crowded lanes, buckets of one and of many segments.  A plain sum of the
+    same terms misses the bound."""
+    val, out, src, x, count, parts = _cancelling(100_003, n_out, 40, dtype.is_complex, n_out)
+    args = [torch.tensor(v, device=DEV) for v in (val, out, src, x)]
+    y = np_(fs.flagsparse_spmv_coo(*args, (n_out, 40)))
+    assert _lib.last_kernel() == "scatter_reduce_kernel"
+    missed = False
+    for got, (ref, mag, plain) in zip((y.real, y.imag), parts):
+        bound = 2.0**-52 * np.abs(ref) + (count * 2.0**-53) ** 2 * mag
+        assert np.all(np.abs(got - ref) <= bound)
+        missed |= bool(np.any(np.abs(plain - ref) > bound))
+    assert missed or n_out > 2500  # (most outputs of 300,007 are one product)
 
 
 # one tile is 6144 entries; 2^8 outputs to a bucket up to 2^18 of them, more beyond
