@@ -21,8 +21,9 @@ _INDEX_LIMIT_INT32 = 2**31 - 1
 
 # Value dtypes every HIP kernel takes.  float16 / bfloat16 are accepted by
 # validation (same messages as the reference), read as they are by the SpMM
-# kernels (_lib.SPMM_HALF_CODES) and converted to float32 elsewhere (the reference's f16/bf16 base path also computes in float32,
-# spmv_csr.py:124-127, spmm_csr.py:2716-2719).
+# kernels (_lib.SPMM_HALF_CODES) and converted to float32 elsewhere (the
+# reference's f16/bf16 base path also computes in float32, spmv_csr.py:124-127,
+# spmm_csr.py:2716-2719).
 HIP_VALUE_DTYPES = (torch.float32, torch.float64, torch.complex64, torch.complex128)
 
 

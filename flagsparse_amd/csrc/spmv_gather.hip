@@ -385,8 +385,8 @@ int launch_gather_spmv(int val_t, int64_t n_rows, int64_t n_cols, int64_t nnz, c
 }
 
 inline bool gather_sizes_ok(int val_t, int64_t n_rows, int64_t n_cols, int64_t nnz) {
-  return val_t >= FS_F32 && val_t < FS_C128 && n_rows > 0 && n_cols > 0 && nnz > 0 && nnz < (int64_t(1) << 31) && n_rows < (int64_t(1) << 31) &&
-         ceil_div(n_cols, int64_t(1) << slice_log2(val_t)) <= kGatherMaxSlices;
+  return val_t >= FS_F32 && val_t < FS_C128 && n_rows > 0 && n_cols > 0 && nnz > 0 && nnz < (int64_t(1) << 31) &&
+         n_rows < (int64_t(1) << 31) && ceil_div(n_cols, int64_t(1) << slice_log2(val_t)) <= kGatherMaxSlices;
 }
 
 }  // namespace fs

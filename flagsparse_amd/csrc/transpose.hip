@@ -1089,11 +1089,11 @@ __global__ __launch_bounds__(kWgThreads, FS_WG_MIN_WAVES) void wg_scatter_kernel
   // without them).
   constexpr bool kWhole = VW == 1;
   if (kWhole && left >= kWgTile)
-    wg_scatter_tile<VW, MODE, kWhole>(keys_in, kind, pay_in, tile, (int)kWgTile, shift, mask, offsets, keys_out, pay_out,
-                                    io, s_buf, s_off, s_wave);
+    wg_scatter_tile<VW, MODE, kWhole>(keys_in, kind, pay_in, tile, (int)kWgTile, shift, mask, offsets, keys_out,
+                                      pay_out, io, s_buf, s_off, s_wave);
   else
-    wg_scatter_tile<VW, MODE, false>(keys_in, kind, pay_in, tile, left < kWgTile ? (int)left : (int)kWgTile, shift, mask, offsets, keys_out, pay_out,
-                                     io, s_buf, s_off, s_wave);
+    wg_scatter_tile<VW, MODE, false>(keys_in, kind, pay_in, tile, left < kWgTile ? (int)left : (int)kWgTile, shift,
+                                     mask, offsets, keys_out, pay_out, io, s_buf, s_off, s_wave);
 }
 
 // colptr[c] = min(colptr[c], colptr[c + 1], ...): block minima, their

@@ -257,9 +257,10 @@ class PreparedCsrSpmv:
 # Column panels (merge-path matrices that the two-phase gather below does not
 # take: complex128, columns beyond its slices, few long rows) pay off once x is
 # larger than an XCD's 4 MiB L2: the random gather rate measured on MI355X drops
-# from ~150-190 to ~70 gathers/ns when x (16.8 MB) no longer fits.  A panel slice of up to ~4.5 MiB measured best
-# (4 panels on a 16.8 MB x: 0.61 ms against 0.67 ms with 8 and 1.01 ms with
-# none) since every panel adds n_rows row ends and partials.
+# from ~150-190 to ~70 gathers/ns when x (16.8 MB) no longer fits.  A panel
+# slice of up to ~4.5 MiB measured best (4 panels on a 16.8 MB x: 0.61 ms against
+# 0.67 ms with 8 and 1.01 ms with none) since every panel adds n_rows row ends
+# and partials.
 _PANEL_X_BYTES = 6 << 20
 _PANEL_SLICE_BYTES = 9 << 19
 
@@ -1468,7 +1469,8 @@ def _spmv_oneshot(data, indices, indptr, x, shape, index_fallback_policy, timed)
     is returned or `out` is written.  Returns (y, compute_ms) or None when
     the general path must run: an invalid x (its error comes after the
     structure checks), empty shapes, float16 / bfloat16 of many entries or
-    long rows, a forced kernel, or a failed launch (the general path holds the int64 -> int32 fallback)."""
+    long rows, a forced kernel, or a failed launch (the general path holds
+    the int64 -> int32 fallback)."""
     if os.environ.get("FLAGSPARSE_SPMV_ONESHOT", "1") == "0" or os.environ.get("FLAGSPARSE_SPMV_KERNEL"):
         return None
     data, indices, indptr, n_rows, n_cols = _validate_spmv_host(data, indices, indptr, shape, index_fallback_policy)
