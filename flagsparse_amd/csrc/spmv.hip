@@ -774,8 +774,9 @@ __global__ __launch_bounds__(256) void spmv_oneshot_kernel(
       // An uneven block, straight from global memory: rows of up to 64 entries
       // by 16 lanes (16 rows at once), up to 4096 by a wave, longer ones by
       // the workgroup.  (Every row by the whole workgroup, with a barrier and
-      // a dependent load and gather for each of 64 rows: R-MAT 2^20 float64 1488
-      // us a call against 1005, 1 M power-law rows float32 277 against 204.)
+      // a dependent load and gather for each of 64 rows: R-MAT 2^20 with 16 entries
+      // a row, float64 1059 us a call against 655, 1 M power-law rows of 16, float32
+      // 233 against 158.)
       constexpr int kShort = 64, kMid = 4096;
       const auto last = ColGuard<I>::last(nc);
       // entries first, first + stride, ... below len of the row at S + a, N loads

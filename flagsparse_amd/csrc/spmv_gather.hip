@@ -19,10 +19,10 @@
 //     entry's 16-bit position.  Products, sums, their order and the fix-up of
 //     rows that span tiles are the merge-path kernel's: the same bits.
 //
-// us per launch, one-pass kernels -> two-phase: power-law 4 M float32 572 -> 335;
-// R-MAT 2^21 float32 291 -> 174, float64 513 -> 332, complex64 605 -> 377; 16
-// uniform columns in each of 4 M rows float32 972 -> 329, float64 1139 -> 632;
-// 1 M rows float32 96 -> 82, float64 187 -> 116.  complex128 gained on none but
+// us per call, one-pass kernels -> two-phase: power-law 4 M float32 563 -> 331;
+// R-MAT 2^21 float32 290 -> 178, float64 513 -> 330, complex64 603 -> 374; 16
+// uniform columns in each of 4,000,000 rows float32 870 -> 315, float64 1057 ->
+// 594; 1 M rows float32 95 -> 82, float64 188 -> 116.  complex128 gained on none but
 // R-MAT 2^21 (283 -> 368 on 1 M uniform rows) and does not take this path.
 //
 // Values are read from the caller's array; the plan holds 5 bytes per entry
@@ -260,7 +260,7 @@ __device__ inline bool region_tile_loads(const V* __restrict__ vals, const uint1
 
 // Phase 2: one region per workgroup.  A wave's first tile is loaded before the
 // region is waited for, and tile i + 1 before tile i is walked.  It moves
-// 4.1 TB/s (power-law 4 M float32: 822 MB in 201 us); with lane tests in whole
+// 4.3 TB/s (power-law 4 M float32: 862 MB in 200 us); with lane tests in whole
 // tiles it was bound by instruction issue (212 us, SIMDs active 88%).
 template <class V, class P>
 __global__ __launch_bounds__(256) void spmv_region_kernel(const V* __restrict__ vals, const uint16_t* __restrict__ pos,

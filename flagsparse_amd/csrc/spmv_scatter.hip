@@ -24,13 +24,13 @@
 // one (product, 16-bit number) pair; the transpose they replace moves (key,
 // value, row) through two passes and ends in a random gather of x.  Both
 // kernels are bound by instruction issue, not by HBM (a 1M x 1M matrix with 32
-// uniform columns per row, float32: 208 + 107 us for 0.5 + 0.17 GB).
+// uniform columns per row, float32: 209 + 108 us for 0.67 + 0.34 GB).
 // Measured, us per call, before (transpose or sort, then SpMV) and now:
-// A^T x of that matrix 889 -> 432; 500,000 rows of 32, complex64 895 -> 468,
-// complex128 1450 -> 490; R-MAT 2^20 complex64 A^H x 1910 -> 710; the 27-point
-// 100^3 stencil, float64, 668 -> 539; 3000 x 2000 ragged, float64, 96 -> 80;
-// COO, 4 M float64 entries over 400,009 rows, 1249 -> 143; 5000 entries over
-// 1000 rows 571 -> 67.
+// A^T x of that matrix 875 -> 394; 500,000 rows of 32, complex64 904 -> 466,
+// complex128 1438 -> 490; R-MAT 2^20 complex64 A^H x 1856 -> 690; the 27-point
+// 100^3 stencil, float64, 674 -> 543; 3000 x 2000 ragged, float64, 93 -> 73;
+// COO, 4 M float64 entries over 400,009 rows, 1180 -> 153; 5000 entries over
+// 1000 rows 607 -> 66.
 //
 // Precision: float32 products are exact in float64 and are summed there, as
 // everywhere else; float64 / complex128 products are rounded once and summed

@@ -1453,8 +1453,8 @@ def _spmv_transposed_oneshot(data, indices, indptr, x, shape, op_code, index_fal
 
 # float16 / bfloat16 take the one-launch call while a call is what counts (us,
 # general path / one launch: 3000 rows of 10 83 / 36, 16,384 of 15 91 / 37);
-# above, hub rows would cost more than its saved launches (R-MAT 2^20: 226 /
-# 816), and so do few long rows, which one workgroup walks (20 rows of 12,000
+# above, hub rows would cost more than its saved launches (R-MAT 2^20: 202 /
+# 568), and so do few long rows, which one workgroup walks (20 rows of 12,000
 # 103 / 222, one of 200,000 102 / 210; one of 60,000 98 / 84, 5 of 13,000 98 /
 # 89): up to 2^16 entries, or 2^18 where rows average at most 64.
 _ONESHOT_HALF_ANY_NNZ = 1 << 16

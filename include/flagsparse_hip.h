@@ -230,7 +230,9 @@ int fs_spmv_csr_oneshot(int val_t, int idx_t, int ptr_t, int64_t n_rows, int64_t
  *     of quads; n_quads its last).
  * fs_spmv_csr_gather: y = A x with slice_q (uint32[ns + 1], the exclusive sum
  * of totals), max_region_quads the largest entry of quads, and ws of
- * fs_spmv_gather_workspace_bytes, used during the call only.
+ * fs_spmv_gather_workspace_bytes, used during the call only.  The gather stores
+ * at places it reads from the plan: a call on another stream than fill's waits
+ * for fill first.
  */
 int fs_spmv_gather_slices(int val_t, int64_t n_rows, int64_t n_cols, int64_t nnz,
                           int64_t* n_regions);
