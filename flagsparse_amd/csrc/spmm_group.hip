@@ -120,6 +120,14 @@ inline int spmm_tile_items_for(int val_t, int64_t n_dense) {
 // 32 160 / 188; 400,009 of 10 174 / 186, 175 / 183; 100,000 of 10 (512 items)
 // 49 / 53, 48 / 52; but 600,000 of 10 (3221 waves) 350 / 293, 44,000 of 50 c128
 // N = 16 99 / 86, and at N = 33 (element loads) 400,009 of 10 289 / 242.
+// With fewer lanes and longer rows 1792 waves are enough: they are nearly two on
+// every SIMD, and halved a round and a half.  us, 2048 waves at least / 1792: rows
+// of 100, 4 M entries f64 N = 16 73 / 67, N = 3 80 / 78, 2 M 42 / 39, 1 M 35 / 24;
+// rows of 1000, 4 M f64 N = 16 80 / 71, f32 N = 32 78 / 72; banded rows of 125, 4 M
+// 87 / 78, 89 / 77.  Not with short rows (500,000 of 6, 1709 waves, f64 N = 16 77
+// halved, 94 not; banded rows of 9 60 / 83) nor on 16-bit values (rows of 30, N =
+// 16 62 / 78), and not with 32 lanes, where halving costs 5% on random columns
+// (rows of 100, 4 M, f32 N = 64 138 / 134) but gains 20% on banded ones (127 / 152).
 constexpr int kGroupMinWaveItems = 128;
 constexpr int64_t kGroupSlots = 3072;
 inline int spmm_tile_items_sized(int val_t, int64_t n_dense, int64_t n_rows, int64_t nnz) {
@@ -127,10 +135,10 @@ inline int spmm_tile_items_sized(int val_t, int64_t n_dense, int64_t n_rows, int
   if (forced_kernel() != 0 || std::getenv("FLAGSPARSE_SPMM_WAVE_ITEMS")) return base;
   if (wide_rows(val_t, n_dense) && nnz >= kGroupSkewNnz) return base;
   const int lpr = group_lpr(val_t, n_dense);
-  const int64_t fill = lpr >= 32 ? 4096 : 2048;
   const int bytes = spmm_value_bytes(val_t);
-  const bool one_round = lpr == 32 && !spmm_half(val_t) && n_dense % (16 / bytes) == 0 &&
-                         nnz / (bytes == 16 ? 12 : 24) <= n_rows;
+  const bool half = spmm_half(val_t), short_rows = nnz / (bytes == 16 ? 12 : 24) <= n_rows;
+  const int64_t fill = lpr >= 32 ? 4096 : half || short_rows ? 2048 : 1792;
+  const bool one_round = lpr == 32 && !half && short_rows && n_dense % (16 / bytes) == 0;
   int wave_items = base * 64 / lpr;
   for (; wave_items > kGroupMinWaveItems; wave_items >>= 1) {
     const int64_t waves = ceil_div(n_rows + nnz, (int64_t)wave_items);

@@ -207,21 +207,19 @@ __global__ __launch_bounds__(256) void scatter_plan_kernel(const uint32_t* __res
   __shared__ int64_t s_wave[4];
   const int q = (nd + 255) / 256;
   const int d0 = threadIdx.x * q;
-  int64_t items = 0, segs = 0, splits = 0;
+  int64_t items = 0, segs = 0;  // segs: segments << 12 | split buckets (at most kWgMaxDigits), one scan for both
   for (int j = 0; j < q; ++j)
     if (d0 + j < nd) {
       const uint32_t c = totals[d0 + j];
-      const uint32_t k = scatter_bucket_segments(c, seg_items);
+      const int64_t k = scatter_bucket_segments(c, seg_items);
       items += c;
-      segs += k;
-      splits += k > 1 ? 1 : 0;
+      segs += k << 12 | (k > 1 ? 1 : 0);
     }
   int64_t all;
   int64_t run = block_exclusive_scan(items, s_wave, all);
   int64_t all_segs;
-  int64_t seg = block_exclusive_scan(segs, s_wave, all_segs);
-  int64_t all_splits;
-  int64_t sp = block_exclusive_scan(splits, s_wave, all_splits);
+  const int64_t first = block_exclusive_scan(segs, s_wave, all_segs);
+  int64_t seg = first >> 12, sp = first & 4095;
   for (int j = 0; j < q; ++j)
     if (d0 + j < nd) {
       const uint32_t c = totals[d0 + j];
@@ -235,8 +233,8 @@ __global__ __launch_bounds__(256) void scatter_plan_kernel(const uint32_t* __res
     }
   if (threadIdx.x == 0) {
     bucket_start[nd] = (uint32_t)all;
-    seg_first[nd] = (uint32_t)all_segs;
-    split[nd] = (uint32_t)all_splits;
+    seg_first[nd] = (uint32_t)(all_segs >> 12);
+    split[nd] = (uint32_t)(all_segs & 4095);
   }
 }
 

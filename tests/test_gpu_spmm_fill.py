@@ -81,6 +81,13 @@ def test_one_round_of_waves_is_not_halved():
     assert size(_lib.FS_F32, 64, 90_000, 4_300_000) == 512  # rows of 48
     assert size(_lib.FS_C128, 16, 400_000, 4_000_000) == 1024
     assert size(_lib.FS_C128, 16, 200_000, 4_000_000) == 512  # rows of 20
+    # 16 lanes a row (a sub-tile is a quarter of a wave's items): 1792 waves of longer rows, 2048 of short ones
+    assert size(_lib.FS_F64, 16, 36_499, 3_649_900) == 512  # 1800 waves of 2048
+    assert size(_lib.FS_F64, 16, 36_093, 3_609_300) == 256  # 1780
+    assert size(_lib.FS_F64, 16, 9_124, 912_400) == 128  # 1800 of 512
+    assert size(_lib.FS_F64, 16, 555_885, 3_335_310) == 256  # 1900, rows of 6
+    assert size(_lib.FS_BF16, 16, 38_526, 3_852_600) == 256  # 1900, 16-bit values
+    assert size(_lib.FS_F32, 64, 41_365, 4_136_500) == 256  # 2040, 32 lanes
 
 
 def test_either_tile_size_is_taken():
