@@ -305,53 +305,54 @@ __global__ __launch_bounds__(256) void spmm_group_kernel(
 // all is a chain of loads that outlasts what small sub-tiles win.  us per
 // prepared float32 call on an arrow matrix of 100,000 rows (its dense row up to
 // 3,125 fragments), 2048-item waves / sized sub-tiles, one wave / 4 waves / 16
-// waves: N = 1 121 / 103 / 25 / 24, N = 17 145 / 142 / 52 / 46, N = 64 178 / 94 /
-// 50 / 43, N = 256 75 / 94 / 71 / 68.  4 waves, and only rows of more than 128
-// fragments: a workgroup of 16 is kept by its slowest wave, and with rows of
-// more than 32 on it the fix-up of an R-MAT graph went from 12 to 18 us (2^19,
-// N = 3, one wave / 4 / 16: 451 / 453 / 455 us a call; 2^21 complex64, N = 32 1393
-// / 1394 / 1396).
+// waves: N = 1 121 / 103 / 24 / 24, N = 17 145 / 142 / 51 / 46, N = 64 178 / 94 /
+// 50 / 43, N = 256 75 / 94 / 71 / 68.  4 waves, as graphs with hubs and the many
+// ordinary rows count for more: the fix-up of R-MAT 2^19, N = 3, one wave / 4 / 16
+// takes 12.4 / 12.3 / 17.6 us, of 2^21 complex64, N = 32 23.0 / 20.4 / 27.9.
 constexpr int kFixWaves = 4;
 constexpr int kFixThreads = 64 * kFixWaves;
 constexpr int64_t kFixShort = 128;
+static_assert((kFixWaves & (kFixWaves - 1)) == 0 && kFixWaves <= kFixShort, "lanes over sub-tiles, one long row");
+__device__ inline int64_t lane_i64(int64_t v, int lane) {
+  return (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), lane) << 32 |
+                   (uint32_t)__builtin_amdgcn_readlane((int)v, lane));
+}
 template <class V, class T = VT<V>>
 __global__ __launch_bounds__(kFixThreads) void spmm_group_fixup_kernel(
     const void* __restrict__ rowptr_raw, int ptr64, const int64_t* __restrict__ part, int sub_items,
     const typename T::acc* __restrict__ head, const typename T::acc* __restrict__ tail,
     V* __restrict__ C, int64_t scm, int64_t scn, int64_t n_dense, int64_t n_sub) {
   using A = typename T::acc;
-  __shared__ int64_t s_long[kFixWaves];  // per wave: the first sub-tile of a long row, or -1
   __shared__ A s_sum[kFixThreads];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int64_t t = (int64_t)blockIdx.x * kFixWaves + (tid >> 6);
-  int64_t long_f = -1;
-  if (t < n_sub) {
-    const int64_t r0 = part[t];
-    const bool ends = part[t + 1] != r0;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t t0 = (int64_t)blockIdx.x * kFixWaves, t = t0 + w;
+  // Every wave finds the workgroup's long row by itself, from loads that go out
+  // with its own: the row that ends in sub-tile k has more than kFixShort
+  // fragments if sub-tile k - kFixShort starts in it.  (A barrier here held every
+  // workgroup for its slowest wave: R-MAT 2^21 bfloat16, N = 3 39 us instead of 30.)
+  const int64_t j = t0 + (lane & (kFixWaves - 1)), k = j < n_sub ? j : n_sub - 1;
+  const int64_t rk = part[k], rk_end = part[k + 1], rk_before = part[k > kFixShort ? k - kFixShort : 0];
+  const uint64_t found =
+      __ballot(lane < kFixWaves && j < n_sub && k > kFixShort && rk_end != rk && rk_before == rk);
+  if (t < n_sub && !((found >> w) & 1)) {
+    const int64_t r0 = lane_i64(rk, w);
+    const bool ends = lane_i64(rk_end, w) != r0;
     const int64_t n0 = t * (int64_t)sub_items - r0;
     const int64_t start = !ends ? n0
                           : ptr64 ? static_cast<const int64_t*>(rowptr_raw)[r0]
                                   : (int64_t) static_cast<const int32_t*>(rowptr_raw)[r0];
     if (start < n0) {
       const int64_t f = fixup_start_tile(part, t, r0);
-      if (t - f > kFixShort) {
-        long_f = f;
-      } else {
-        for (int64_t col = (int64_t)blockIdx.y * 64 + lane; col < n_dense; col += (int64_t)gridDim.y * 64) {
-          A sum = tail[f * n_dense + col];
-          sum = sum_fragments(tail + col, n_dense, f + 1, t, sum);  // in sub-tile order
-          sum = add(sum, head[t * n_dense + col]);
-          C[r0 * scm + col * scn] = T::out(sum);
-        }
+      for (int64_t col = (int64_t)blockIdx.y * 64 + lane; col < n_dense; col += (int64_t)gridDim.y * 64) {
+        A sum = tail[f * n_dense + col];
+        sum = sum_fragments(tail + col, n_dense, f + 1, t, sum);  // in sub-tile order
+        sum = add(sum, head[t * n_dense + col]);
+        C[r0 * scm + col * scn] = T::out(sum);
       }
     }
   }
-  if (lane == 0) s_long[tid >> 6] = long_f;
-  __syncthreads();
-  const uint64_t found = __ballot(lane < kFixWaves && s_long[lane < kFixWaves ? lane : 0] >= 0);
   if (found == 0) return;  // whole workgroup
-  const int lw = (int)__builtin_ctzll(found);
-  const int64_t lt = (int64_t)blockIdx.x * kFixWaves + lw, lf = s_long[lw], row = part[lt];
+  const int64_t lt = t0 + (int)__builtin_ctzll(found), row = part[lt], lf = fixup_start_tile(part, lt, row);
   for (int64_t c0 = (int64_t)blockIdx.y * 64; c0 < n_dense; c0 += (int64_t)gridDim.y * 64) {
     const int nc = n_dense - c0 < 64 ? (int)(n_dense - c0) : 64;
     int width = 1;  // threads per share: the columns, rounded up to a power of two
