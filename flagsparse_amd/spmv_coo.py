@@ -254,15 +254,18 @@ class _PreparedCooLaunch:
         "sorted",
         "conj",
         "bad_indices",
+        "scatter_bytes",
     )
 
     # sorted_coo: the sorted orientation, or None for a launch over the caller's
-    # unsorted entries, which leaves (bad row, bad col) in bad_indices.
+    # unsorted entries, whose workspace takes scatter_bytes and which leaves
+    # (bad row, bad col) in bad_indices.
     def __init__(self, sorted_coo, data, row, col, shape, seg_starts=None, op=SPMV_COO_OP_NON, conj=False,
                  index_fallback_policy="auto", index_fallback_applied=False, index_fallback_reason=None):
         self.sorted = sorted_coo
         self.conj = bool(conj)
         self.bad_indices = None
+        self.scatter_bytes = 0
         self.data = data
         self.row = row
         self.col = col
@@ -374,13 +377,17 @@ def _spmv_coo_prepared_with_int32_indices(launch, reason):
         raise RuntimeError(f"native int64 COO SpMV failed and int32 fallback is unsafe: {blocker}")
     seg = None if launch.seg_starts is None else launch.seg_starts.to(torch.int32).contiguous()
     srt = launch.sorted
-    sorted32 = None if srt is None else _SortedCoo(srt.data, srt.row.to(torch.int32), srt.col.to(torch.int32),
-                          None if srt.seg_starts is None else srt.seg_starts.to(torch.int32), srt.indptr.to(torch.int32),
-                          srt.shape)
-    return _PreparedCooLaunch(sorted32, launch.data, launch.row.to(torch.int32).contiguous(),
-                              launch.col.to(torch.int32).contiguous(), launch.shape, seg_starts=seg, op=launch.op,
-                              conj=launch.conj, index_fallback_policy=launch.index_fallback_policy,
-                              index_fallback_applied=True, index_fallback_reason=str(reason))
+    sorted32 = None
+    if srt is not None:
+        seg32 = None if srt.seg_starts is None else srt.seg_starts.to(torch.int32)
+        sorted32 = _SortedCoo(srt.data, srt.row.to(torch.int32), srt.col.to(torch.int32), seg32,
+                              srt.indptr.to(torch.int32), srt.shape)
+    fallback = _PreparedCooLaunch(sorted32, launch.data, launch.row.to(torch.int32).contiguous(),
+                                  launch.col.to(torch.int32).contiguous(), launch.shape, seg_starts=seg, op=launch.op,
+                                  conj=launch.conj, index_fallback_policy=launch.index_fallback_policy,
+                                  index_fallback_applied=True, index_fallback_reason=str(reason))
+    fallback.scatter_bytes = launch.scatter_bytes
+    return fallback
 
 
 def _run_spmv_coo_prepared_with_fallback(launch, x, block_size, num_warps, block_inner):
@@ -487,7 +494,7 @@ def _hip_spmv_coo_scatter(launch, x):
     val_t = _lib.value_code(launch.data.dtype)
     device = launch.data.device
     y = torch.empty(launch.n_rows, dtype=launch.data.dtype, device=device)
-    ws = _lib.workspace(lib.fs_spmv_scatter_workspace_bytes(val_t, launch.n_rows, launch.nnz), device)
+    ws = _lib.workspace(launch.scatter_bytes, device)
     flags = _oneshot_flags()
     _lib.check(
         lib.fs_spmv_coo_scatter(
@@ -529,13 +536,16 @@ def _spmv_coo_unsorted(data, row, col, x, shape, op_code, block_size, num_warps,
         or num_warps not in (1, 2, 4, 8, 16, 32)
         or block_inner <= 0
         or (block_inner & (block_inner - 1)) != 0
-        or _lib.lib().fs_spmv_scatter_workspace_bytes(_lib.value_code(data.dtype), n_out, data.numel()) == 0
     ):
+        return None
+    ws_bytes = _lib.lib().fs_spmv_scatter_workspace_bytes(_lib.value_code(data.dtype), n_out, data.numel())
+    if ws_bytes == 0:
         return None
     out_idx, x_idx = (col, row) if transposes else (row, col)
     launch = _PreparedCooLaunch(None, data.contiguous(), out_idx.contiguous(), x_idx.contiguous(), (n_out, n_x),
                                 op=op_code, conj=op_code == SPMV_COO_OP_CONJ_TRANS and data.dtype.is_complex,
                                 index_fallback_policy=index_fallback_policy)
+    launch.scatter_bytes = ws_bytes
     x = x.contiguous()
     if timed:
         torch.cuda.synchronize()

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import flagsparse_amd as fs
-from flagsparse_amd import _lib
+from flagsparse_amd import _lib, spmv_coo
 from flagsparse_amd import synthetic as S
 from oracle import csr_oracle as O
 from tests._helpers import INDEX_DTYPES, INDEX_IDS, REL_TOL, VALUE_DTYPES, VALUE_IDS, np_, rel_err
@@ -251,3 +251,23 @@ def test_row_pointers_of_any_value_are_refused(value, n_cols):
     p[100] = value
     with pytest.raises(ValueError, match="non-decreasing"):
         fs.flagsparse_spmv_csr(d, i, p, S.vector(300, torch.float32, DEV, 4), (300, n_cols), op="trans")
+
+
+def test_coo_failed_int64_call_runs_again_on_int32_indices(monkeypatch):
+    data, row, col = _coo(5000, 300, 200, torch.float64, torch.int64, torch.int64, 4)
+    x = S.vector(200, torch.float64, DEV, 2)
+    y = fs.flagsparse_spmv_coo(data, row, col, x, (300, 200))
+    kernel, tried = spmv_coo._hip_spmv_coo_scatter, []
+
+    def fails_on_int64(launch, x):
+        tried.append(launch.row.dtype)
+        if launch.row.dtype == torch.int64:
+            raise RuntimeError("refused")
+        return kernel(launch, x)
+
+    monkeypatch.setattr(spmv_coo, "_hip_spmv_coo_scatter", fails_on_int64)
+    assert torch.equal(fs.flagsparse_spmv_coo(data, row, col, x, (300, 200)), y)
+    assert tried == [torch.int64, torch.int32]
+    row[3] = 300
+    with pytest.raises(IndexError, match="row indices"):
+        fs.flagsparse_spmv_coo(data, row, col, x, (300, 200))
